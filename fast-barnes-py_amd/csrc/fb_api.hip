@@ -486,11 +486,12 @@ struct fb_plan {
     int64_t *d_pt_prefix = nullptr, *d_xline_prefix = nullptr, *d_cell_prefix = nullptr;
     int64_t *d_lslot_prefix[3] = {nullptr, nullptr, nullptr};
     int64_t lslots[3] = {0, 0, 0};
-    // FP64 x lines through LDS (k_exact_rows): first workgroup of each field, workgroups in
-    // all, slots per workgroup, and the widest x kernel (2T+1) of the fields
-    int64_t *d_rowwg_prefix = nullptr;
-    int64_t rowwgs = 0, row_rect = 0;
-    int row_slots = 64;
+    // FP64 lines through LDS (k_exact_stream), per axis: the geometry (ni = 0: k_exact_lines takes
+    // the axis), first workgroup of each field, workgroups in all; the fields' most iterations
+    LineGeom lgeom[3];
+    int64_t *d_lwg_prefix[3] = {nullptr, nullptr, nullptr};
+    int64_t lwgs[3] = {0, 0, 0};
+    int max_iter = 0;
     double *d_offsets = nullptr, *d_off_part = nullptr;
     int64_t max_n = 0;
     int64_t max_rows = 0;   // most x-lines of any field
@@ -915,7 +916,8 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     P->corners = 1 << P->dim;
     const int fast = precision == FB_PREC_FP32C;
     P->fh.resize(nfields);
-    std::vector<int64_t> pt_prefix, xline_prefix, cell_prefix, lslot[3], rowwg;
+    std::vector<int64_t> pt_prefix, xline_prefix, cell_prefix, lslot[3], lwg[3];
+    int64_t max_rect[3] = {1, 1, 1}, max_len[3] = {1, 1, 1};
     for (int f = 0; f < nfields; ++f) {
         int rc = make_field(fields[f], P->fh[f], fast);
         if (rc) { delete P; return rc; }
@@ -936,7 +938,11 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
             lslot[a].push_back(P->lslots[a]);
             if (a < P->dim) P->lslots[a] += 2 * nl[a];
         }
-        P->row_rect = std::max(P->row_rect, 2 * (int64_t)d.T[0] + 1);
+        for (int a = 0; a < 3; ++a) {
+            max_rect[a] = std::max(max_rect[a], 2 * (int64_t)d.T[a] + 1);
+            max_len[a] = std::max(max_len[a], d.size[a]);
+        }
+        P->max_iter = std::max(P->max_iter, d.num_iter);
         P->npoints += d.n;
         P->nxlines += H * D;
         // 256-byte aligned field starts (float4 tiles); an FP32C 2D field that may keep its
@@ -950,12 +956,15 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     xline_prefix.push_back(P->nxlines);
     cell_prefix.push_back(P->ncells);
     for (int a = 0; a < 3; ++a) lslot[a].push_back(P->lslots[a]);
-    P->row_slots = exact_rows_slots(P->lslots[0]);
-    for (const FieldDev &d : P->fh) {
-        rowwg.push_back(P->rowwgs);
-        P->rowwgs += (2 * d.size[1] * d.size[2] + P->row_slots - 1) / P->row_slots;
+    for (int a = 0; a < P->dim && !fast; ++a) {
+        P->lgeom[a] = line_geom(max_rect[a], P->max_iter, max_len[a]);
+        const int64_t lines = P->lgeom[a].ni ? kLineSlots / 2 : 1;
+        for (const FieldDev &d : P->fh) {
+            lwg[a].push_back(P->lwgs[a]);
+            P->lwgs[a] += (d.size[0] * d.size[1] * d.size[2] / d.size[a] + lines - 1) / lines;
+        }
+        lwg[a].push_back(P->lwgs[a]);
     }
-    rowwg.push_back(P->rowwgs);
     P->nentries = P->npoints;   // one (base cell, point) pair per point
     if (P->ncells >= (int64_t)kInvalidKey || P->npoints >= (int64_t)UINT32_MAX || P->nentries >= (int64_t)UINT32_MAX) {
         delete P;
@@ -971,7 +980,8 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
         TRY(P->upload_all({item(&P->d_fields, P->fh), item(&P->d_pt_prefix, pt_prefix),
                            item(&P->d_xline_prefix, xline_prefix), item(&P->d_cell_prefix, cell_prefix),
                            item(&P->d_lslot_prefix[0], lslot[0]), item(&P->d_lslot_prefix[1], lslot[1]),
-                           item(&P->d_lslot_prefix[2], lslot[2]), item(&P->d_rowwg_prefix, rowwg)}));
+                           item(&P->d_lslot_prefix[2], lslot[2]), item(&P->d_lwg_prefix[0], lwg[0]),
+                           item(&P->d_lwg_prefix[1], lwg[1]), item(&P->d_lwg_prefix[2], lwg[2])}));
     }
     TRY(P->alloc(&P->d_offsets, nfields));
     for (const FieldDev &d : P->fh) {
@@ -997,8 +1007,12 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     } else if (!fast) {
         TRY(P->alloc(&P->d_vg, P->ncells));
         TRY(P->alloc(&P->d_wg, P->ncells));
-        TRY(P->alloc(&P->d_vs, P->ncells));
-        TRY(P->alloc(&P->d_ws, P->ncells));
+        bool wide = false;   // an axis for k_exact_lines, which needs the second pair of planes
+        for (int a = 0; a < P->dim; ++a) wide = wide || !P->lgeom[a].ni;
+        if (wide) {
+            TRY(P->alloc(&P->d_vs, P->ncells));
+            TRY(P->alloc(&P->d_ws, P->ncells));
+        }
         TRY(P->alloc(&P->d_irec, P->npoints));
     } else {
         TRY(P->alloc(&P->d_v, P->ncells));
@@ -1088,16 +1102,18 @@ int plan_run(fb_plan *P, const double *pts, const double *val, float *out, float
         stage_mark(P, s, "inject");
         static const char *ln[3] = {"lines_x", "lines_y", "lines_z"};
         for (int a = 0; a < P->dim; ++a) {
-            if (a == 0 && exact_rows_ring(P->row_rect))
-                rc = launch_exact_rows(P->d_fields, P->d_rowwg_prefix, P->d_lslot_prefix[0], P->nfields, P->rowwgs,
-                                       P->row_slots, -1, P->row_rect, P->d_vg, P->d_wg, P->d_vs, P->d_ws, s);
+            const LineGeom &g = P->lgeom[a];
+            if (g.ni)   // the last axis leaves the float32 result
+                rc = launch_exact_stream(P->d_fields, P->d_lwg_prefix[a], P->nfields, P->lwgs[a], a, -1, g, P->max_iter,
+                                         P->d_vg, P->d_wg, P->d_offsets, a == P->dim - 1 ? out : nullptr, s);
             else
                 rc = launch_exact_lines(P->d_fields, P->d_lslot_prefix[a], P->nfields, P->lslots[a], a, -1, P->d_vg,
                                         P->d_wg, P->d_vs, P->d_ws, s);
             if (rc) return rc;
             stage_mark(P, s, ln[a]);
         }
-        if ((rc = launch_exact_finalize(P->d_fields, P->d_cell_prefix, P->nfields, P->ncells, P->d_vg, P->d_wg,
+        if (!P->lgeom[P->dim - 1].ni &&
+            (rc = launch_exact_finalize(P->d_fields, P->d_cell_prefix, P->nfields, P->ncells, P->d_vg, P->d_wg,
                                         P->d_offsets, out, s)))
             return rc;
         stage_mark(P, s, "finalize");
@@ -2002,19 +2018,20 @@ int fb_accumulate_lines(int tail, int precision, int64_t nlines, int64_t len, in
     if (precision == FB_PREC_FP64) {
         double *d_w, *d_vs, *d_ws;
         int64_t *d_pre;
-        if ((rc = sc.get(&d_w, cells)) || (rc = sc.get(&d_vs, cells)) || (rc = sc.get(&d_ws, cells)) ||
-            (rc = sc.get(&d_pre, 4)))
-            return rc;
+        if ((rc = sc.get(&d_w, cells)) || (rc = sc.get(&d_pre, 4))) return rc;
         if ((rc = launch_zero(d_w, cells * 8, s))) return rc;
-        if ((rc = fast_pass_init())) return rc;   // k_exact_rows' LDS limit
-        // line slots, then the x-line workgroups of k_exact_rows
-        const int sl = exact_rows_slots(2 * nlines);
-        const int64_t nwg = (2 * nlines + sl - 1) / sl;
+        if ((rc = fast_pass_init())) return rc;   // the line kernels' LDS limit
+        // line slots, then the workgroups of k_exact_stream
+        const LineGeom g = line_geom(rect_len, num_iter, len);
+        const int64_t per = g.ni ? kLineSlots / 2 : 1, nwg = (nlines + per - 1) / per;
         const int64_t pre[4] = {0, 2 * nlines, 0, nwg};
         FB_HIP_CHECK(hipMemcpy(d_pre, pre, sizeof(pre), hipMemcpyHostToDevice));
-        rc = exact_rows_ring(rect_len)
-                 ? launch_exact_rows(d_f, d_pre + 2, d_pre, 1, nwg, sl, rect_len, rect_len, d_io, d_w, d_vs, d_ws, s)
-                 : launch_exact_lines(d_f, d_pre, 1, 2 * nlines, 0, rect_len, d_io, d_w, d_vs, d_ws, s);
+        if (g.ni) {
+            rc = launch_exact_stream(d_f, d_pre + 2, 1, nwg, 0, rect_len, g, num_iter, d_io, d_w, nullptr, nullptr, s);
+        } else {
+            if ((rc = sc.get(&d_vs, cells)) || (rc = sc.get(&d_ws, cells))) return rc;
+            rc = launch_exact_lines(d_f, d_pre, 1, 2 * nlines, 0, rect_len, d_io, d_w, d_vs, d_ws, s);
+        }
         if (rc) return rc;
     } else {
         if (rect_len % 2 == 0) return fail(FB_ERR_UNSUPPORTED, "FP32C line passes need an odd rect_len");
@@ -2109,20 +2126,22 @@ int fb_convolve_grid(int tail, int precision, int dim, const int64_t *size, cons
     const int64_t W = F.size[0], H = F.size[1], D = F.size[2];
     const int64_t nl[3] = {H * D, W * D, W * H};
     if (precision == FB_PREC_FP64) {
-        double *d_vs, *d_ws;
+        double *d_vs = nullptr, *d_ws = nullptr;
         int64_t *d_pre;
-        if ((rc = sc.get(&d_vs, cells)) || (rc = sc.get(&d_ws, cells)) || (rc = sc.get(&d_pre, 4))) return rc;
-        if ((rc = fast_pass_init())) return rc;   // k_exact_rows' LDS limit
+        if ((rc = sc.get(&d_pre, 4))) return rc;
+        if ((rc = fast_pass_init())) return rc;   // the line kernels' LDS limit
         for (int a = 0; a < dim; ++a) {
-            // line slots, then (x lines) the workgroups of k_exact_rows
-            const int sl = exact_rows_slots(2 * nl[a]);
-            const int64_t nwg = (2 * nl[a] + sl - 1) / sl;
+            // line slots, then the workgroups of k_exact_stream
+            const LineGeom g = line_geom(2 * (int64_t)F.T[a] + 1, num_iter, F.size[a]);
+            const int64_t per = g.ni ? kLineSlots / 2 : 1, nwg = (nl[a] + per - 1) / per;
             const int64_t pre[4] = {0, 2 * nl[a], 0, nwg};
-            const int64_t rect = 2 * (int64_t)F.T[0] + 1;
             FB_HIP_CHECK(hipMemcpy(d_pre, pre, sizeof(pre), hipMemcpyHostToDevice));
-            rc = a == 0 && exact_rows_ring(rect)
-                     ? launch_exact_rows(d_f, d_pre + 2, d_pre, 1, nwg, sl, -1, rect, d_vg, d_wg, d_vs, d_ws, s)
-                     : launch_exact_lines(d_f, d_pre, 1, 2 * nl[a], a, -1, d_vg, d_wg, d_vs, d_ws, s);
+            if (g.ni) {
+                rc = launch_exact_stream(d_f, d_pre + 2, 1, nwg, a, -1, g, num_iter, d_vg, d_wg, nullptr, nullptr, s);
+            } else {
+                if (!d_vs && ((rc = sc.get(&d_vs, cells)) || (rc = sc.get(&d_ws, cells)))) return rc;
+                rc = launch_exact_lines(d_f, d_pre, 1, 2 * nl[a], a, -1, d_vg, d_wg, d_vs, d_ws, s);
+            }
             if (rc) return rc;
             FB_HIP_CHECK(hipStreamSynchronize(s));   // d_pre is reused by the next axis
         }

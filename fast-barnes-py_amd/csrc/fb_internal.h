@@ -14,6 +14,17 @@ constexpr uint32_t kInvalidKey = 0xFFFFFFFFu;
 // largest field (points) the per-field LDS sort takes (64-bit entries: 64 KiB of LDS)
 constexpr int kLocalSortMax = 8192;
 
+// largest f in [0, n) with prefix[f] <= i
+__device__ __forceinline__ int find_seg(const int64_t *__restrict__ prefix, int n, int64_t i)
+{
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (prefix[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
 // Per-field descriptor as the kernels see it.  Everything is derived on the host in
 // FP64 from the reference's own formulas, except the value offset, which the
 // offset kernel computes on the device into a separate array.
@@ -126,36 +137,45 @@ struct PointRec {
     int32_t pad_;
 };
 
-// FP64 x lines through LDS (k_exact_rows): tiles of kRowTile columns, a ring of `ring` tiles
-// per (line, field) slot, 32 or 64 slots per workgroup.  exact_rows_ring: the ring's tiles for
-// a kernel of rect terms (0 when a 64-slot workgroup's ring would not fit the LDS);
-// exact_rows_lds: the bytes of a workgroup of `slots` slots.
-constexpr int kRowTile = 32;
-// mir: the ring's first kRowTile + 1 positions repeated past its end, so that a chunk's reads
-// never wrap (slot stride odd either way)
-__host__ __device__ inline int64_t exact_rows_slot_stride(int ring, bool mir = false)
+// FP64 line passes through LDS rings (k_exact_stream): kLineStep steps per tick for kLineSlots
+// slots (lines x {v, w}); the iterations share waves, 64 / kLineSlots to a wave, and three more
+// waves load and store.
+constexpr int kLineStep = 16;
+constexpr int kLineSlots = 16;
+constexpr int kLineIterMax = 8;                   // iterations of one launch
+constexpr int kLineWavesMax = kLineIterMax * kLineSlots / 64 + 3;
+constexpr int kLineLdsMax = 160 * 1024;
+
+// doubles of one ring of R blocks and its first block again (pairs of positions, kLineSlots + 1
+// apart)
+__host__ __device__ inline int line_ring_doubles(int R) { return (R + 1) * kLineStep * (kLineSlots + 1); }
+
+// ni: iterations per launch, R: blocks per ring
+struct LineGeom {
+    int ni = 0, R = 0;
+    size_t lds = 0;
+};
+
+// Geometry for kernels of up to max_rect terms and max_iter iterations: the ring holds the
+// blocks that an iteration reads (h1 positions back, h0 + 1 ahead) and the one its predecessor
+// writes; as many iterations per launch as the LDS takes.  ni = 0: not even one, or lines of
+// length max_len > 2^30 (the kernel's positions are 32-bit); k_exact_lines takes such lines.
+inline LineGeom line_geom(int64_t max_rect, int max_iter, int64_t max_len)
 {
-    return (int64_t)ring * kRowTile + (mir ? kRowTile + 1 : 1);
-}
-__host__ __device__ inline int64_t exact_rows_lds(int ring, int slots, bool mir = false)
-{
-    return (slots * exact_rows_slot_stride(ring, mir) + slots * (kRowTile + 1)) * (int64_t)sizeof(double);
-}
-inline int exact_rows_ring(int64_t rect)
-{
-    const int64_t h0 = (rect - 1) / 2, h1 = rect - h0;
-    const int64_t need = h0 / kRowTile + (h1 + kRowTile - 1) / kRowTile + 2;
-    int ring = 1;
-    while (ring < need) ring <<= 1;
-    return exact_rows_lds(ring, 64) <= 160 * 1024 ? ring : 0;
-}
-// slots per workgroup of k_exact_rows for a plan of `slots` x-line slots: 64, or 32 or 16
-// while fewer than 256 workgroups (one per CU of an MI355X) would take the lines
-inline int exact_rows_slots(int64_t slots)
-{
-    int s = 64;
-    while (s > 16 && (slots + s - 1) / s < 256) s >>= 1;
-    return s;
+    LineGeom g;
+    if (max_len > (1 << 30)) return g;
+    const int64_t h0 = (max_rect - 1) / 2, h1 = max_rect - h0;
+    const int64_t R = (h1 + kLineStep - 1) / kLineStep + h0 / kLineStep + 3;
+    const int64_t want = max_iter < 1 ? 1 : max_iter < kLineIterMax ? max_iter : kLineIterMax;
+    const int64_t out = 2 * kLineStep * (kLineSlots + 1) * (int64_t)sizeof(double);
+    if (R > (1 << 20)) return g;
+    const int64_t ring = line_ring_doubles((int)R) * (int64_t)sizeof(double);
+    const int64_t fit = (kLineLdsMax - out) / ring;
+    if (fit < 1) return g;
+    g.ni = (int)(fit < want ? fit : want);
+    g.R = (int)R;
+    g.lds = (size_t)(g.ni * ring + out);
+    return g;
 }
 
 // FP64 injection: one sorted entry's record (k_inject_records), in list order.
