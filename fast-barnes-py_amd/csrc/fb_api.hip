@@ -1096,8 +1096,8 @@ int plan_run(fb_plan *P, const double *pts, const double *val, float *out, float
         if ((rc = launch_inject_records(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints,
                                         P->max_n <= kLocalSortMax, P->nxlines, vs, P->d_line_start,
                                         P->d_line_count, pts, val, P->d_offsets, P->d_irec, s)) ||
-            (rc = launch_exact_inject(P->d_fields, P->d_xline_prefix, P->nfields, P->nxlines, P->d_irec,
-                                      P->d_line_start, P->d_line_count, P->d_vg, P->d_wg, P->dim, true, s)))
+            (rc = launch_inject_cells(P->d_fields, P->npoints, P->d_irec, P->d_line_start, P->d_line_count, P->d_vg,
+                                      P->d_wg, P->dim, true, s)))
             return rc;
         stage_mark(P, s, "inject");
         static const char *ln[3] = {"lines_x", "lines_y", "lines_z"};
@@ -1852,8 +1852,8 @@ int fb_inject(int dim, int64_t n, const double *pts, const double *val, const do
                                    P->nxlines, vs, P->d_line_start, P->d_line_count, d_pts, d_val, P->d_offsets,
                                    P->d_irec, s);
     if (!rc)
-        rc = launch_exact_inject(P->d_fields, P->d_xline_prefix, 1, P->nxlines, P->d_irec, P->d_line_start,
-                                 P->d_line_count, d_vg, d_wg, P->dim, false, s);
+        rc = launch_inject_cells(P->d_fields, P->npoints, P->d_irec, P->d_line_start, P->d_line_count, d_vg, d_wg,
+                                 P->dim, false, s);
     if (!rc && !on_dev) {
         if (hipMemcpyAsync(vg, d_vg, cells * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipMemcpyAsync(wg, d_wg, cells * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) {

@@ -182,6 +182,8 @@ inline LineGeom line_geom(int64_t max_rect, int max_iter, int64_t max_len)
 struct InjectRec {
     int x;              // base column
     uint32_t p;         // point index
+    uint32_t row;       // base row (x-line index of the plan); kInvalidKey: no entry
+    int f;              // field
     double wx, wy, wz;  // position within the base cell
     double vc;          // value minus the field's offset
 };

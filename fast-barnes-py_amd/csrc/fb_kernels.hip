@@ -6,7 +6,7 @@
 //                   per-row point counts                          interpolation.py:218-322
 //   (fb_sort.hip)   scan of the row counts; per-field LDS sort or row buckets ordering the
 //                   pairs by (base cell, point index)
-//   FP64 path:      k_exact_inject, k_exact_stream (fb_lines.hip) along each axis, the last one
+//   FP64 path:      k_inject_cells, k_exact_stream (fb_lines.hip) along each axis, the last one
 //                   with the quotient -- the reference's operation order; k_exact_lines (one
 //                   thread per line) and k_exact_finalize for kernels too wide for the LDS
 //   FP32C path:     k_fast_pass<inject> along x, k_fast_pass along y (and z);
@@ -422,11 +422,11 @@ __device__ __forceinline__ void line_streams(const FieldDev &F, int64_t line, bo
 // ---------------------------------------------------------------------------
 // FP64 path, reference operation order
 
-// Each sorted entry's injection record, in list order (the merge then reads one record per
-// step): base column, point, position within the base cell and value minus the offset, as
-// point_pos forms them.  The per-field sort (`local`) writes a field's in-grid points from its
-// first point index on and leaves the slots after them unused; the row-bucket sort packs all
-// fields' entries by row.  Slots past the list's last entry are skipped.
+// Each sorted entry's injection record, in list order: base column and row, point, field,
+// position within the base cell and value minus the offset, as point_pos forms them.  The
+// per-field sort (`local`) writes a field's in-grid points from its first point index on and
+// leaves the slots after them unused; the row-bucket sort packs all fields' entries by row.  Slots
+// past the list's last entry get row kInvalidKey.
 __global__ __launch_bounds__(kBlock) void k_inject_records(
     const FieldDev *__restrict__ fields, const int64_t *__restrict__ pt_prefix, int nfields, int64_t npoints,
     int local, int64_t nxlines, const uint32_t *__restrict__ vals, const uint32_t *__restrict__ row_start,
@@ -440,195 +440,123 @@ __global__ __launch_bounds__(kBlock) void k_inject_records(
         const FieldDev &Fe = fields[find_seg(pt_prefix, nfields, e)];
         last = Fe.xline_off + Fe.size[1] * Fe.size[2] - 1;   // the last row of the slot's field
     }
-    if (e >= (int64_t)row_start[last] + row_count[last]) return;
+    if (e >= (int64_t)row_start[last] + row_count[last]) {
+        irec[e].row = kInvalidKey;
+        return;
+    }
     const uint32_t p = vals[e];
     const int f = find_seg(pt_prefix, nfields, p);
     const FieldDev &F = fields[f];
     PointPos pp;
     point_pos(F, pts + (int64_t)p * F.dim, pp);
-    irec[e] = InjectRec{(int)pp.i[0], p, pp.w[0], pp.w[1], pp.w[2], val[p] - offsets[f]};
+    irec[e] = InjectRec{(int)pp.i[0], p, (uint32_t)(F.xline_off + pp.i[2] * F.size[1] + pp.i[1]), f,
+                        pp.w[0], pp.w[1], pp.w[2], val[p] - offsets[f]};
 }
 
-// One thread per x-line: merges the line's sub-streams by (x, point index) and adds
-// w*val_c and w to the FP64 grids in that order, which is the per-cell order of the
-// reference's point loop (each cell gets its contributions in increasing point index).
-// The contributions of a cell are consecutive in the merged order, so a cell's two sums are
-// held in registers and stored once; they start at 0.0 when the grids were cleared (zeroed),
-// else at the grids' values.  One wave per workgroup, as k_exact_lines: a field has only as
-// many threads as x lines.
+// The injection, cell by cell: a grid cell t receives corner s (its bits: x, y, z) of the points of
+// base cell t - s, s < 2^DIM, in increasing point index, which is the order of the reference's
+// point loop.  One thread per sorted entry and corner: the first entry of a base cell's run takes
+// the cell at that corner of it, unless a base cell of a smaller s has points too (then that one's
+// thread takes it), finds the runs of the cell's other base cells in their rows by bisection, all
+// of them in step, and merges the runs by point index.  The cell's sums start at 0.0 when the grids
+// were cleared (ZEROED), else at the grids' values, and are stored once.
 //
-// The merge is a chain of dependent steps, one entry record read per step.  When a
-// workgroup's lines lie in one 1D or 2D field and their rows (each line's own and, in 2D,
-// the row below) hold at most stage_cap points, the wave first copies those records to LDS
-// (dynamic, stage_cap records: kInjectStage for plans of 1D and 2D fields, none for 3D) and
-// the merge reads them there.  A field's rows are contiguous in the sorted list (each
-// row starts where the previous one ends), so the workgroup's records are one range of it.
-constexpr int kExactInjectThreads = 64;
-constexpr int kInjectStage = 1024;
-
-// head of sub-stream q at entry e: target x, point, corner weight, value (x = INT_MAX when
-// the stream is exhausted); STAGED reads the record from LDS.  q may differ between the
-// lanes: its corner (q & 1, (q >> 1) & 1, q >> 2) selects the weight's factors.
-template <bool STAGED>
-__device__ __forceinline__ void inject_head(const FieldDev &F, int q, uint32_t e, uint32_t end,
-                                            const InjectRec *rec, uint32_t e0,
-                                            const InjectRec *__restrict__ irec, int &x, uint32_t &p,
-                                            double &w, double &v)
+// Bound by latency: about six reads per bisection, one per contribution, each depending on the one
+// before.  A thread per x line that merged the rows' entries took as long as the line had entries:
+// 3490 points on 300x150 (23 to a row) 139 us, here 12; on 2400x1200 27 us, here 8; 20000 on
+// 151x133x61 73 us, here 17; 24 fields of 3490 on 600x300 99 us, here 16.
+template <int DIM, bool ZEROED>
+__global__ __launch_bounds__(kBlock) void k_inject_cells(
+    const FieldDev *__restrict__ fields, int64_t npoints, const InjectRec *__restrict__ irec,
+    const uint32_t *__restrict__ row_start, const uint32_t *__restrict__ row_count, double *__restrict__ vg,
+    double *__restrict__ wg)
 {
-    if (e >= end) {
-        x = INT_MAX;
-        p = 0;
-        w = v = 0.0;
-        return;
-    }
-    const InjectRec &r = STAGED ? rec[e - e0] : irec[e];
-    PointPos pp;
-    pp.i[0] = r.x;
-    pp.i[1] = pp.i[2] = 0;
-    pp.w[0] = r.wx;
-    pp.w[1] = r.wy;
-    pp.w[2] = r.wz;
-    p = r.p;
-    v = r.vc;
-    x = r.x + (q & 1);
-    w = corner_weight(F.dim, pp, q & 1, (q >> 1) & 1, q >> 2);
-}
+    constexpr int NC = 1 << DIM;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t e = (uint32_t)(i >> DIM);
+    if ((i >> DIM) >= npoints) return;
+    const int own = (int)i & (NC - 1);
+    const uint32_t row = irec[e].row;
+    if (row == kInvalidKey) return;
+    const int bx = irec[e].x;
+    const FieldDev &F = fields[irec[e].f];
+    const uint32_t rs = row_start[row];
+    if (e > rs && irec[e - 1].x == bx) return;
+    const int64_t H = F.size[1], lrow = (int64_t)row - F.xline_off;
+    const int64_t y = DIM >= 3 ? (uint32_t)lrow % (uint32_t)H : lrow;   // a 2D line is its row
+    const int64_t z = DIM >= 3 ? (uint32_t)lrow / (uint32_t)H : 0;
 
-// the merge of one line's NS sub-streams (4 in 1D and 2D, 8 in 3D).  Each step takes the
-// smallest head and reads the next entry of that stream only: one read per step whichever
-// stream each lane advances.  A cell's sums start at 0.0 (ZEROED) or at the grids' values,
-// and are stored when the merge moves past the cell.
-template <int NS, bool STAGED, bool ZEROED>
-__device__ __forceinline__ void inject_merge(const FieldDev &F, uint32_t (&pos)[8], const uint32_t (&end)[8],
-                                             const InjectRec *rec, uint32_t e0,
-                                             const InjectRec *__restrict__ irec, double *__restrict__ vg,
-                                             double *__restrict__ wg, int64_t base)
-{
-    // hr: entries left in the stream after its head (loop-carried, like the heads, so that
-    // taking the advanced stream's values stays a chain of selects, not an indexed array)
-    uint32_t hp[NS], hr[NS];
-    int hx[NS];
-    double hw[NS], hv[NS];
+    // the sources' rows; source s starts at its first entry of column tx - (s & 1) or beyond
+    const int tx = bx + (own & 1);
+    uint32_t lo[NC], end[NC];
 #pragma unroll
-    for (int q = 0; q < NS; ++q) {
-        inject_head<STAGED>(F, q, pos[q], end[q], rec, e0, irec, hx[q], hp[q], hw[q], hv[q]);
-        hr[q] = pos[q] < end[q] ? end[q] - pos[q] - 1 : 0;
+    for (int s = 0; s < NC; ++s) {
+        const int dy = ((own >> 1) & 1) - ((s >> 1) & 1), dz = (own >> 2) - (s >> 2);
+        lo[s] = end[s] = 0;
+        if (tx - (s & 1) >= 0 && y + dy >= 0 && z + dz >= 0) {
+            const uint32_t r = (uint32_t)((int64_t)row + dy + dz * H);
+            lo[s] = row_start[r];
+            end[s] = lo[s] + row_count[r];
+        }
     }
-    int cx = INT_MAX;
-    double av = 0.0, aw = 0.0;
+    uint32_t hi[NC];
+#pragma unroll
+    for (int s = 0; s < NC; ++s) {
+        hi[s] = end[s];
+        if (s == own) lo[s] = hi[s] = e;
+    }
+    for (bool more = true; more;) {
+        more = false;
+#pragma unroll
+        for (int s = 0; s < NC; ++s) {
+            if (lo[s] < hi[s]) {
+                const uint32_t mid = (lo[s] + hi[s]) >> 1;
+                if (irec[mid].x < tx - (s & 1)) lo[s] = mid + 1;
+                else hi[s] = mid;
+                more = more || lo[s] < hi[s];
+            }
+        }
+    }
+    // the next entry's point of each source, kInvalidKey when the run has ended
+    uint32_t head[NC];
+#pragma unroll
+    for (int s = 0; s < NC; ++s) {
+        head[s] = lo[s] < end[s] && irec[lo[s]].x == tx - (s & 1) ? irec[lo[s]].p : kInvalidKey;
+        if (s < own && head[s] != kInvalidKey) return;
+    }
+    const int64_t cell = F.cell_off + tx + (int64_t)F.size[0] * (lrow + ((own >> 1) & 1) + (own >> 2) * H);
+    double av = ZEROED ? 0.0 : vg[cell];
+    double aw = ZEROED ? 0.0 : wg[cell];
     while (true) {
         int best = 0;
+        uint32_t p = head[0], at = lo[0], stop = end[0];
 #pragma unroll
-        for (int q = 1; q < NS; ++q)
-            if (hx[q] < hx[best] || (hx[q] == hx[best] && hp[q] < hp[best])) best = q;
-        int bx = hx[0];
-        double bw = hw[0], bv = hv[0];
-        uint32_t e = pos[0] + 1, r = hr[0];
-#pragma unroll
-        for (int q = 1; q < NS; ++q)
-            if (q == best) {
-                bx = hx[q];
-                bw = hw[q];
-                bv = hv[q];
-                e = pos[q] + 1;
-                r = hr[q];
+        for (int s = 1; s < NC; ++s)
+            if (head[s] < p) {
+                best = s;
+                p = head[s];
+                at = lo[s];
+                stop = end[s];
             }
-        // every stream exhausted (at once for a line without points): store the last cell
-        if (bx == INT_MAX) {
-            if (cx != INT_MAX) {
-                vg[base + cx] = av;
-                wg[base + cx] = aw;
-            }
-            break;
-        }
-        int nx;
-        uint32_t np;
-        double nw, nv;
-        inject_head<STAGED>(F, best, e, r ? e + 1 : e, rec, e0, irec, nx, np, nw, nv);
+        if (p == kInvalidKey) break;
+        const InjectRec &r = irec[at];
+        const uint32_t nx = at + 1 < stop && irec[at + 1].x == r.x ? irec[at + 1].p : kInvalidKey;
+        PointPos pp;
+        pp.w[0] = r.wx;
+        pp.w[1] = r.wy;
+        pp.w[2] = r.wz;
+        const double w = corner_weight(DIM, pp, best & 1, (best >> 1) & 1, best >> 2);
+        av += w * r.vc;
+        aw += w;
 #pragma unroll
-        for (int q = 0; q < NS; ++q)
-            if (q == best) {
-                pos[q] = e;
-                hr[q] = r ? r - 1 : 0;
-                hx[q] = nx;
-                hp[q] = np;
-                hw[q] = nw;
-                hv[q] = nv;
+        for (int s = 0; s < NC; ++s)
+            if (s == best) {
+                head[s] = nx;
+                lo[s] = at + 1;
             }
-        if (bx != cx) {
-            if (cx != INT_MAX) {
-                vg[base + cx] = av;
-                wg[base + cx] = aw;
-            }
-            cx = bx;
-            av = ZEROED ? 0.0 : vg[base + cx];
-            aw = ZEROED ? 0.0 : wg[base + cx];
-        }
-        av += bw * bv;
-        aw += bw;
     }
-}
-
-__global__ __launch_bounds__(kExactInjectThreads) void k_exact_inject(
-    const FieldDev *__restrict__ fields, const int64_t *__restrict__ xline_prefix, int nfields, int64_t nxlines,
-    const InjectRec *__restrict__ irec, const uint32_t *__restrict__ row_start,
-    const uint32_t *__restrict__ row_count, double *__restrict__ vg, double *__restrict__ wg, int zeroed,
-    int stage_cap)
-{
-    extern __shared__ InjectRec rec[];
-    const int64_t g0 = (int64_t)blockIdx.x * kExactInjectThreads;
-    const int64_t glast = min(g0 + kExactInjectThreads - 1, nxlines - 1);
-    const int64_t gl = g0 + threadIdx.x;
-    const bool live = gl < nxlines;
-    const int f = find_seg(xline_prefix, nfields, live ? gl : glast);
-    const FieldDev &F = fields[f];
-    const int64_t line = (live ? gl : glast) - F.xline_off;
-    const int64_t base = F.cell_off + line * F.size[0];
-    uint32_t pos[8], end[8];
-    {
-        uint32_t rs[8], rc[8];
-        line_streams(F, line, live, row_start, row_count, rs, rc);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            pos[q] = rs[q];
-            end[q] = rs[q] + rc[q];
-        }
-    }
-    // stage the workgroup's records when its lines share one 1D/2D field (then F is the same
-    // for every lane and both conditions are uniform) and every stream lies in their range
-    bool staged = false;
-    uint32_t e0 = 0;
-    if (find_seg(xline_prefix, nfields, g0) == find_seg(xline_prefix, nfields, glast) && F.dim <= 2) {
-        const int64_t lo = (F.dim == 2 && g0 > F.xline_off) ? g0 - 1 : g0;
-        e0 = row_start[lo];
-        const uint32_t e1 = row_start[glast] + row_count[glast];
-        bool ok = e0 <= e1 && e1 - e0 <= (uint32_t)stage_cap;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) ok = ok && (pos[q] == end[q] || (pos[q] >= e0 && end[q] <= e1));
-        staged = __all(ok);
-        if (staged) {
-            for (uint32_t e = e0 + threadIdx.x; e < e1; e += kExactInjectThreads) rec[e - e0] = irec[e];
-            __syncthreads();
-        }
-    }
-    if (!live) return;
-    // staged lines are 1D or 2D (4 streams)
-    if (staged) {
-        if (zeroed)
-            inject_merge<4, true, true>(F, pos, end, rec, e0, irec, vg, wg, base);
-        else
-            inject_merge<4, true, false>(F, pos, end, rec, e0, irec, vg, wg, base);
-    } else if (F.dim <= 2) {
-        if (zeroed)
-            inject_merge<4, false, true>(F, pos, end, rec, e0, irec, vg, wg, base);
-        else
-            inject_merge<4, false, false>(F, pos, end, rec, e0, irec, vg, wg, base);
-    } else {
-        if (zeroed)
-            inject_merge<8, false, true>(F, pos, end, rec, e0, irec, vg, wg, base);
-        else
-            inject_merge<8, false, false>(F, pos, end, rec, e0, irec, vg, wg, base);
-    }
+    vg[cell] = av;
+    wg[cell] = aw;
 }
 
 // _accumulate_tail_array (interpolation.py:484-533) and _accumulate_array (:729-772)
@@ -2039,19 +1967,30 @@ int launch_inject_records(const FieldDev *d_fields, const int64_t *d_pt_prefix, 
     return FB_OK;
 }
 
-int launch_exact_inject(const FieldDev *d_fields, const int64_t *d_xline_prefix, int nfields, int64_t nxlines,
-                        const InjectRec *d_irec, const uint32_t *d_row_start, const uint32_t *d_row_count,
-                        double *d_vg, double *d_wg, int dim, bool zeroed, hipStream_t s)
+int launch_inject_cells(const FieldDev *d_fields, int64_t npoints, const InjectRec *d_irec,
+                        const uint32_t *d_row_start, const uint32_t *d_row_count, double *d_vg, double *d_wg, int dim,
+                        bool zeroed, hipStream_t s)
 {
-    if (nxlines <= 0) return FB_OK;
+    if (npoints <= 0) return FB_OK;
     if (!d_irec) {
         set_error("FP64 injection: the plan has no record array");
         return FB_ERR_INVALID_ARGUMENT;
     }
-    const int cap = dim <= 2 ? kInjectStage : 0;   // 3D lines never stage
-    hipLaunchKernelGGL(k_exact_inject, dim3((unsigned)((nxlines + kExactInjectThreads - 1) / kExactInjectThreads)),
-                       dim3(kExactInjectThreads), (size_t)cap * sizeof(InjectRec), s, d_fields, d_xline_prefix,
-                       nfields, nxlines, d_irec, d_row_start, d_row_count, d_vg, d_wg, zeroed ? 1 : 0, cap);
+    const dim3 grid((unsigned)(((npoints << dim) + kBlock - 1) / kBlock)), block(kBlock);
+#define FB_CELLS(D_, Z_)                                                                                          \
+    hipLaunchKernelGGL((k_inject_cells<D_, Z_>), grid, block, 0, s, d_fields, npoints, d_irec, d_row_start, d_row_count, \
+                       d_vg, d_wg)
+    if (dim == 1) {
+        if (zeroed) FB_CELLS(1, true);
+        else FB_CELLS(1, false);
+    } else if (dim == 2) {
+        if (zeroed) FB_CELLS(2, true);
+        else FB_CELLS(2, false);
+    } else {
+        if (zeroed) FB_CELLS(3, true);
+        else FB_CELLS(3, false);
+    }
+#undef FB_CELLS
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
