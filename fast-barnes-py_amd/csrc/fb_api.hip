@@ -1901,8 +1901,12 @@ int fb_barnes(int method, int precision, int dim, int64_t n, const double *pts, 
             const double radius = std::sqrt(-2.0 * std::log(min_weight)) * sigma[0];
             r2 = radius * radius;
         }
-        if ((rc = launch_naive(d_f, method == FB_METHOD_RADIUS, r2, max_dist_weight, d_pts, d_val, d_off, d_out,
-                               cells, s)))
+        const int radius = method == FB_METHOD_RADIUS;
+        double *d_work = nullptr;
+        if (const int64_t elems = naive_work_elems(radius, dim, F.size, n))
+            if (sc.get(&d_work, elems)) d_work = nullptr;   // no memory for the tables: node by node
+        if ((rc = launch_naive(d_f, radius, r2, max_dist_weight, dim, F.size, n, d_pts, d_val, d_off, d_work, d_out,
+                               s)))
             return rc;
         if (!on_dev) FB_HIP_CHECK(stage.down(out, d_out, cells * sizeof(double)));
         FB_HIP_CHECK(hipStreamSynchronize(s));

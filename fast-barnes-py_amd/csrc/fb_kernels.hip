@@ -1735,78 +1735,6 @@ __global__ __launch_bounds__(kBlock) void k_f32_to_f64(const float *__restrict__
 }
 
 // ---------------------------------------------------------------------------
-// naive (interpolation.py:861-938) and radius (:809-855, brute force in place of the
-// kd-tree, same inclusion test sqr_dist <= radius^2) in FP64, one thread per node.
-
-__global__ __launch_bounds__(kBlock) void k_naive(const FieldDev *__restrict__ fp, int radius, double r2, double mdw,
-                                                  const double *__restrict__ pts, const double *__restrict__ val,
-                                                  const double *__restrict__ offsets, double *__restrict__ out,
-                                                  int64_t ncells)
-{
-    __shared__ double sp[3][kBlock];
-    __shared__ double sval[kBlock];
-    const FieldDev F = *fp;
-    const int tid = threadIdx.x;
-    const int64_t g = (int64_t)blockIdx.x * kBlock + tid;
-    const int dim = F.dim;
-    const int64_t W = F.size[0], H = F.size[1];
-    const int64_t x = g % W, y = (g / W) % H, z = g / (W * H);
-    const double c0 = F.x0[0] + (double)x * F.step[0];
-    const double c1 = dim > 1 ? F.x0[1] + (double)y * F.step[1] : 0.0;
-    const double c2 = dim > 2 ? F.x0[2] + (double)z * F.step[2] : 0.0;
-    // scale = 2*sigma**2 per axis (interpolation.py:872)
-    const double s0 = 2 * (F.sigma[0] * F.sigma[0]);
-    const double s1 = 2 * (F.sigma[1] * F.sigma[1]);
-    const double s2 = 2 * (F.sigma[2] * F.sigma[2]);
-    const double off = offsets[0];
-    double ws = 0.0, wt = 0.0;
-    for (int64_t b = 0; b < F.n; b += kBlock) {
-        __syncthreads();
-        const int64_t k = b + tid;
-        if (k < F.n) {
-            for (int m = 0; m < dim; ++m) sp[m][tid] = pts[k * dim + m];
-            sval[tid] = val[k] - off;
-        }
-        __syncthreads();
-        const int cnt = (int)min((int64_t)kBlock, F.n - b);
-        if (g < ncells) {
-            if (!radius) {
-                for (int t = 0; t < cnt; ++t) {
-                    const double d0 = sp[0][t] - c0;
-                    double d = d0 * d0 / s0;
-                    if (dim > 1) {
-                        const double d1 = sp[1][t] - c1;
-                        d = d + d1 * d1 / s1;
-                    }
-                    if (dim > 2) {
-                        const double d2 = sp[2][t] - c2;
-                        d = d + d2 * d2 / s2;
-                    }
-                    const double w = exp(-d);
-                    ws += w * sval[t];
-                    wt += w;
-                }
-            } else {
-                for (int t = 0; t < cnt; ++t) {
-                    const double dx = c0 - sp[0][t];
-                    const double dy = c1 - sp[1][t];
-                    const double d2 = dx * dx + dy * dy;
-                    if (d2 <= r2) {
-                        const double w = exp(-d2 / s0);
-                        ws += w * sval[t];
-                        wt += w;
-                    }
-                }
-            }
-        }
-    }
-    if (g < ncells) {
-        if (!radius) out[g] = wt > 0.0 ? ws / wt + off : __builtin_nan("");
-        else out[g] = wt >= mdw ? ws / wt + off : __builtin_nan("");
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Adjoint of the FP32C batch (no counterpart in the reference, which has no gradient).
 //
 // On unmasked nodes f = V/W + offset with V = B S (val - offset), W = B S 1, where S is
@@ -2157,16 +2085,6 @@ int launch_f32_to_f64(const float *in, double *out, int64_t n, double scale, hip
 {
     if (n <= 0) return FB_OK;
     hipLaunchKernelGGL(k_f32_to_f64, dim3(nblocks(n)), dim3(kBlock), 0, s, in, out, n, scale);
-    FB_HIP_CHECK(hipGetLastError());
-    return FB_OK;
-}
-
-int launch_naive(const FieldDev *d_field, int radius, double radius_sqr, double max_dist_weight, const double *d_pts,
-                 const double *d_val, const double *d_offsets, double *d_out, int64_t ncells, hipStream_t s)
-{
-    if (ncells <= 0) return FB_OK;
-    hipLaunchKernelGGL(k_naive, dim3(nblocks(ncells)), dim3(kBlock), 0, s, d_field, radius, radius_sqr,
-                       max_dist_weight, d_pts, d_val, d_offsets, d_out, ncells);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }

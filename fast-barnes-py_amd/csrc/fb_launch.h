@@ -113,9 +113,11 @@ int launch_zero(void *p, int64_t bytes, hipStream_t stream);   // bytes: multipl
 int launch_f64_to_f32(const double *in, float *out, int64_t n, hipStream_t stream);
 int launch_f32_to_f64(const float *in, double *out, int64_t n, double scale, hipStream_t stream);
 
-// fb_kernels.hip -- naive / radius (O(N*W*H*D) brute force, FP64)
-int launch_naive(const FieldDev *d_field, int radius, double radius_sqr, double max_dist_weight,
-                 const double *d_pts, const double *d_val, const double *d_offsets, double *d_out, int64_t ncells,
-                 hipStream_t stream);
+// fb_naive.hip -- naive / radius sums in FP64.  naive_work_elems: doubles of workspace with which
+// the naive sums run as matrix products (0: node by node); with d_work = NULL they run node by node.
+int64_t naive_work_elems(int radius, int dim, const int64_t *size, int64_t n);
+int launch_naive(const FieldDev *d_field, int radius, double radius_sqr, double max_dist_weight, int dim,
+                 const int64_t *size, int64_t n, const double *d_pts, const double *d_val, const double *d_offsets,
+                 double *d_work, double *d_out, hipStream_t stream);
 
 }  // namespace fb
