@@ -645,7 +645,7 @@ struct fb_plan {
     int device = 0;
     int precision = FB_PREC_FP64;
     int nfields = 0, dim = 0, corners = 0;
-    int64_t npoints = 0, ncells = 0, nxlines = 0, nentries = 0, total_out = 0, total_cells = 0;
+    int64_t npoints = 0, ncells = 0, nxlines = 0, total_out = 0, total_cells = 0;
     std::vector<FieldDev> fh;
     std::vector<DevBuf> bufs;
     size_t ws_bytes = 0;
@@ -663,9 +663,12 @@ struct fb_plan {
     double *d_offsets = nullptr, *d_off_part = nullptr;
     int64_t max_n = 0;
     int64_t max_rows = 0;   // most x-lines of any field
-    uint32_t *d_keys = nullptr, *d_vals = nullptr, *d_keys2 = nullptr, *d_vals2 = nullptr;
-    uint32_t *d_line_count = nullptr, *d_line_start = nullptr, *d_scan_tmp = nullptr;
-    uint32_t *d_skeys = nullptr, *d_big_list = nullptr, *d_big_count = nullptr;   // row buckets
+    bool local = false;     // k_field_sort takes the sort stage of every field; else row buckets
+    uint32_t *d_list = nullptr;                                 // the sorted point list
+    uint32_t *d_keys = nullptr, *d_slot = nullptr;              // row buckets: base cells, slots,
+    unsigned long long *d_comp = nullptr;                       // entries by row, scan tiles and counter
+    uint32_t *d_tiles = nullptr, *d_done = nullptr;
+    uint32_t *d_line_count = nullptr, *d_line_start = nullptr;
     PointRec *d_rec = nullptr;                  // FP32C: each point's position for the injection
     InjectRec *d_irec = nullptr;                // FP64: each sorted entry's injection record
     double *d_vg = nullptr, *d_wg = nullptr, *d_vs = nullptr, *d_ws = nullptr;
@@ -674,7 +677,6 @@ struct fb_plan {
     PassField *d_pass[3] = {nullptr, nullptr, nullptr};
     std::vector<PassGroup> groups[3];          // launches of each axis pass, one per segment length
     std::map<std::pair<int, int64_t>, PassChoice> seg_choice;   // (axis, line length) -> autotuned choice
-    const uint32_t *sorted_vals = nullptr;      // sorted point indices of the last run
     int allow_blocked = 1;                      // fb_plan_set_blocked
     bool inplace_passes = false;                // every pass filters its planes in place (no chunks)
 
@@ -1139,8 +1141,7 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
         }
         lwg[a].push_back(P->lwgs[a]);
     }
-    P->nentries = P->npoints;   // one (base cell, point) pair per point
-    if (P->ncells >= (int64_t)kInvalidKey || P->npoints >= (int64_t)UINT32_MAX || P->nentries >= (int64_t)UINT32_MAX) {
+    if (P->ncells >= (int64_t)kInvalidKey || P->npoints >= (int64_t)UINT32_MAX) {
         delete P;
         return fail(FB_ERR_UNSUPPORTED, "a plan holds at most 2^32-2 grid cells and 2^32-1 contributions");
     }
@@ -1162,32 +1163,45 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
         P->max_n = std::max(P->max_n, d.n);
         P->max_rows = std::max(P->max_rows, d.size[1] * d.size[2]);
     }
+    // One workgroup per field sorts fields of few points and rows; beyond, a workgroup per field would
+    // walk them alone (5000 points on 100x90x60, 5400 rows: 86 us, the row buckets 28).
+    P->local = P->max_n <= kLocalSortMax && P->max_rows <= kLocalRowsMax;
+    const bool records = !fast;   // the FP64 injection reads its records, the FP32C x pass the list
     TRY(P->alloc(&P->d_off_part, offsets_part_elems(nfields, P->max_n)));
-    TRY(P->alloc(&P->d_keys, P->nentries));
-    TRY(P->alloc(&P->d_vals, P->nentries));
-    TRY(P->alloc(&P->d_keys2, P->nentries));
-    TRY(P->alloc(&P->d_vals2, P->nentries));
-    if (P->max_n > kLocalSortMax) {
-        TRY(P->alloc(&P->d_skeys, P->nentries));
-        TRY(P->alloc(&P->d_big_list, 2 * P->nxlines));   // rows for the wave kernel, then larger rows
-        TRY(P->alloc(&P->d_big_count, 2));
+    if (records) TRY(P->alloc(&P->d_irec, P->npoints));
+    if (!P->local) {
+        // keys, slots and composites are spent when the records are written and share their
+        // memory; without records the list takes the keys' place
+        if (records) {
+            P->d_comp = (unsigned long long *)P->d_irec;
+            P->d_keys = (uint32_t *)(P->d_comp + P->npoints);
+            P->d_slot = P->d_keys + P->npoints;
+            static_assert(sizeof(InjectRec) >= 16, "the sort's arrays fit the records");
+            TRY(P->alloc(&P->d_list, P->npoints));
+        } else {
+            TRY(P->alloc(&P->d_comp, P->npoints));
+            TRY(P->alloc(&P->d_keys, P->npoints));
+            TRY(P->alloc(&P->d_slot, P->npoints));
+            P->d_list = P->d_keys;
+        }
+        TRY(P->alloc(&P->d_tiles, scan_tiles(P->nxlines) + 1));
+        P->d_done = P->d_tiles + scan_tiles(P->nxlines);
+    } else if (!records) {
+        TRY(P->alloc(&P->d_list, P->npoints));
     }
     TRY(P->alloc(&P->d_line_count, P->nxlines));
     TRY(P->alloc(&P->d_line_start, P->nxlines));
-    TRY(P->alloc(&P->d_scan_tmp, scan_temp_elems(P->nxlines)));
     if (!grids) {
         // the sort and injection stages only (fb_inject): the caller's grids take the sums
-        TRY(P->alloc(&P->d_irec, P->npoints));
     } else if (!fast) {
         TRY(P->alloc(&P->d_vg, P->ncells));
         TRY(P->alloc(&P->d_wg, P->ncells));
         bool wide = false;   // an axis for k_exact_lines, which needs the second pair of planes
         for (int a = 0; a < P->dim; ++a) wide = wide || !P->lgeom[a].ni;
-        if (wide) {
+        if (wide || arena) {   // the fixed scratch counts them always: its limit is one of sizes only
             TRY(P->alloc(&P->d_vs, P->ncells));
             TRY(P->alloc(&P->d_ws, P->ncells));
         }
-        TRY(P->alloc(&P->d_irec, P->npoints));
     } else {
         TRY(P->alloc(&P->d_v, P->ncells));
         TRY(P->alloc(&P->d_w, P->ncells));
@@ -1210,48 +1224,31 @@ void stage_mark(fb_plan *P, hipStream_t s, const char *name)
     P->stage_names.push_back(name);
 }
 
-// The sort stage of a run: the value offsets and the points ordered by base row, (base cell,
-// point index); *sorted receives the sorted point indices.
-int plan_sort(fb_plan *P, const double *pts, const double *val, hipStream_t s, const uint32_t **sorted)
+// The sort stage of a run: the value offsets (zeros with `raw`), the rows' counts and starts, and the
+// points ordered by base row, (base cell, point index): the point list and each point's record of an
+// FP32C plan, the injection records of an FP64 plan, whose grids are zeroed as well.
+int plan_sort(fb_plan *P, const double *pts, const double *val, bool raw, hipStream_t s)
 {
     int rc;
-    // Per-row point counts by integer atomics and their exclusive scan give the rows' ranges of
-    // the sorted list.  Fields of at most kLocalSortMax points: one workgroup sorts each field
-    // in LDS.  Larger fields: every point goes to its atomic slot of its row's range, then each
-    // row is sorted by (key, point index).  Both give the order of a stable sort of the (key,
-    // point index) pairs.
-    const bool local = P->max_n <= kLocalSortMax;
-    if ((rc = launch_zero(P->d_line_count, P->nxlines * 4, s))) return rc;
-    if (!local && (rc = launch_zero(P->d_big_count, 8, s))) return rc;
-    if (offsets_single_pass(P->max_n, P->d_off_part)) {
-        if ((rc = launch_point_keys_offsets(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, pts, P->d_keys,
-                                            P->d_vals, P->d_line_count, local ? nullptr : P->d_vals,
-                                            local ? nullptr : P->d_keys2, val, P->d_offsets, P->d_rec, s)))
-            return rc;
-    } else {
-        if ((rc = launch_offsets(P->d_fields, P->nfields, P->max_n, val, P->d_off_part, P->d_offsets, s))) return rc;
-        if ((rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, pts, P->d_keys, P->d_vals,
-                                    P->d_line_count, local ? nullptr : P->d_vals, local ? nullptr : P->d_keys2, P->max_rows, P->d_rec, s)))
-            return rc;
-    }
-    uint32_t *vs = P->d_vals2;
-    if (local) {
-        // the field sort scans each field's row counts itself (a field's list starts at its
-        // first point index)
-        if ((rc = launch_field_sort(P->d_fields, P->d_pt_prefix, P->nfields, (int)P->max_n, P->d_keys,
-                                    P->d_line_count, P->d_line_start, P->d_vals2, s)))
-            return rc;
-    } else {
-        if ((rc = scan_exclusive(P->d_line_count, P->d_line_start, P->nxlines, P->d_scan_tmp, s))) return rc;
-        // d_vals holds the slots and d_keys2 the rows; both, with d_keys, are free after the
-        // scatter and serve as scratch for rows of more than kLocalSortMax points
-        if ((rc = row_bucket_sort(P->d_keys, P->d_vals, P->d_keys2, P->npoints, P->d_line_start, P->d_line_count,
-                                  P->nxlines, P->d_skeys, P->d_vals2, P->d_big_list, P->d_big_count, P->d_keys,
-                                  P->d_vals, s)))
-            return rc;
-    }
-    *sorted = vs;
-    return FB_OK;
+    const ZeroRange vg{(uint4 *)P->d_vg, P->d_vg ? P->ncells / 2 : 0};   // ncells is a multiple of 64
+    const ZeroRange wg{(uint4 *)P->d_wg, P->d_wg ? P->ncells / 2 : 0};
+    if (P->local)
+        return launch_field_sort(P->d_fields, P->d_pt_prefix, P->nfields, P->dim, (int)P->max_n, (int)P->max_rows, pts,
+                                 val, raw, P->d_offsets, P->d_line_count, P->d_line_start, P->d_list, P->d_rec,
+                                 P->d_irec, {vg, wg}, s);
+    // whole 16-byte words: the row counts' allocation is a multiple of 256 bytes
+    const ZeroRange counts{(uint4 *)P->d_line_count, (P->nxlines + 3) / 4};
+    if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->max_n, val, P->d_off_part, P->d_done, {counts, vg, wg}, s)) ||
+        (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->max_n, P->npoints, pts, P->d_keys,
+                                P->d_line_count, P->d_slot, P->max_rows, P->d_rec, P->d_off_part, P->d_offsets, s)) ||
+        (rc = row_bucket_sort(P->d_fields, P->d_pt_prefix, P->nfields, P->d_keys, P->d_slot, P->npoints,
+                              P->d_line_start, P->d_line_count, P->nxlines, P->d_tiles, P->d_done, P->d_comp, P->d_list,
+                              s)))
+        return rc;
+    if (!P->d_irec) return FB_OK;
+    if (raw && (rc = launch_zero(P->d_offsets, P->nfields * 8, s))) return rc;
+    return launch_inject_records(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, P->nxlines, P->d_list,
+                                 P->d_line_start, P->d_line_count, pts, val, P->d_offsets, P->d_irec, s);
 }
 
 int plan_run(fb_plan *P, const double *pts, const double *val, float *out, float *wsave, hipStream_t s)
@@ -1261,17 +1258,10 @@ int plan_run(fb_plan *P, const double *pts, const double *val, float *out, float
     P->events.clear();
     P->stage_names.clear();
     stage_mark(P, s, "begin");
-    const uint32_t *vs = nullptr;
-    if ((rc = plan_sort(P, pts, val, s, &vs))) return rc;
-    P->sorted_vals = vs;
+    if ((rc = plan_sort(P, pts, val, false, s))) return rc;
     stage_mark(P, s, "sort");
     if (P->precision == FB_PREC_FP64) {
-        if ((rc = launch_zero(P->d_vg, P->ncells * 8, s))) return rc;
-        if ((rc = launch_zero(P->d_wg, P->ncells * 8, s))) return rc;
-        if ((rc = launch_inject_records(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints,
-                                        P->max_n <= kLocalSortMax, P->nxlines, vs, P->d_line_start,
-                                        P->d_line_count, pts, val, P->d_offsets, P->d_irec, s)) ||
-            (rc = launch_inject_cells(P->d_fields, P->npoints, P->d_irec, P->d_line_start, P->d_line_count, P->d_vg,
+        if ((rc = launch_inject_cells(P->d_fields, P->npoints, P->d_irec, P->d_line_start, P->d_line_count, P->d_vg,
                                       P->d_wg, P->dim, true, s)))
             return rc;
         stage_mark(P, s, "inject");
@@ -1296,7 +1286,7 @@ int plan_run(fb_plan *P, const double *pts, const double *val, float *out, float
         static const char *pn[3] = {"pass_x", "pass_y", "pass_z"};
         for (int a = 0; a < P->dim; ++a) {
             const int fin = a == P->dim - 1;
-            if ((rc = run_pass(P, a, a == 0, vs, val, out, fin ? wsave : nullptr, fin, s))) return rc;
+            if ((rc = run_pass(P, a, a == 0, P->d_list, val, out, fin ? wsave : nullptr, fin, s))) return rc;
             stage_mark(P, s, pn[a]);
         }
     }
@@ -1566,7 +1556,7 @@ static int time_pass(fb_plan *P, int a, const std::vector<PassWork> &fw, const s
         if (rep == 1) (void)hipEventRecord(e0, s);
         for (const PassGroup &g : fg) {
             rc = launch_fast_pass(g.kind, a == 0, g.seg, P->d_fields, P->d_offsets, dw + g.first, g.count, dp, 2 * g.lpf,
-                                  g.lds, P->d_rec, P->sorted_vals, P->d_line_start, P->d_line_count, val, P->d_v,
+                                  g.lds, P->d_rec, P->d_list, P->d_line_start, P->d_line_count, val, P->d_v,
                                   P->d_w, out, nullptr, fin, nullptr, s);
             if (rc) break;
         }
@@ -2019,18 +2009,9 @@ int fb_inject(int dim, int64_t n, const double *pts, const double *val, const do
     const fb_field f = single_field(FB_METHOD_OPTIMIZED_CONVOLUTION, dim, n, sig, x0, step, size, 1, 0.0);
     fb_plan *P = nullptr;
     if ((rc = plan_create(&P, &f, 1, FB_PREC_FP64, nullptr, 0, false))) return rc;
-    const uint32_t *vs = nullptr;
-    rc = plan_sort(P, d_pts, d_val, s, &vs);
     // the values are injected as given: offset 0 (one field's grid starts at cell 0, x-fastest,
     // exactly the caller's layout)
-    if (!rc && hipMemsetAsync(P->d_offsets, 0, sizeof(double), s) != hipSuccess) {
-        (void)hipGetLastError();
-        rc = fail(FB_ERR_HIP, "clearing the offset failed");
-    }
-    if (!rc)
-        rc = launch_inject_records(P->d_fields, P->d_pt_prefix, 1, P->npoints, P->max_n <= kLocalSortMax,
-                                   P->nxlines, vs, P->d_line_start, P->d_line_count, d_pts, d_val, P->d_offsets,
-                                   P->d_irec, s);
+    rc = plan_sort(P, d_pts, d_val, true, s);
     if (!rc)
         rc = launch_inject_cells(P->d_fields, P->npoints, P->d_irec, P->d_line_start, P->d_line_count, d_vg, d_wg,
                                  P->dim, false, s);

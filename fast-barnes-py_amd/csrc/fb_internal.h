@@ -11,8 +11,15 @@ namespace fb {
 // Sentinel sort key of a contribution that falls outside the grid
 // (reference: the `continue` of interpolation.py:226,249,283).
 constexpr uint32_t kInvalidKey = 0xFFFFFFFFu;
-// largest field (points) the per-field LDS sort takes (64-bit entries: 64 KiB of LDS)
+// largest field (points, x-lines) the per-field LDS sort takes (64-bit entries: 64 KiB of LDS)
 constexpr int kLocalSortMax = 8192;
+constexpr int kLocalRowsMax = 4096;
+
+// 16-byte words from p on that a kernel zeroes
+struct ZeroRange {
+    uint4 *p;
+    int64_t n;
+};
 
 // largest f in [0, n) with prefix[f] <= i
 __device__ __forceinline__ int find_seg(const int64_t *__restrict__ prefix, int n, int64_t i)
@@ -186,12 +193,6 @@ struct InjectRec {
     int f;              // field
     double wx, wy, wz;  // position within the base cell
     double vc;          // value minus the field's offset
-};
-
-// Contribution record of the sorted injection list.
-struct Contrib {
-    uint32_t key;          // global cell index (kInvalidKey when outside)
-    uint32_t pidx;         // global point index
 };
 
 }  // namespace fb

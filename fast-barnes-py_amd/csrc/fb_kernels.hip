@@ -1,22 +1,23 @@
 // fb_kernels.hip -- device kernels of fast Barnes interpolation on gfx950.
 //
 // Pipeline of one batch (every stage covers all fields of the batch):
-//   k_offsets       value offset (min+max)/2 per field           interpolation.py:204-212
-//   k_point_keys    per point: base cell (lower corner) -> (cell key, point) pair,
-//                   per-row point counts                          interpolation.py:218-322
-//   (fb_sort.hip)   scan of the row counts; per-field LDS sort or row buckets ordering the
-//                   pairs by (base cell, point index)
+//   sort stage      value offset (min+max)/2 per field           interpolation.py:204-212
+//                   and the points in (base cell, point index) order, interpolation.py:218-322: fields of
+//                   few points in one launch (k_field_sort, fb_sort.hip); larger ones k_sort_begin,
+//                   k_point_keys (cells and row counts), then the row buckets of fb_sort.hip
 //   FP64 path:      k_inject_cells, k_exact_stream (fb_lines.hip) along each axis, the last one
 //                   with the quotient -- the reference's operation order; k_exact_lines (one
 //                   thread per line) and k_exact_finalize for kernels too wide for the LDS
 //   FP32C path:     k_fast_pass<inject> along x, k_fast_pass along y (and z);
 //                   quotient, offset and NaN mask fused into the last pass
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <mutex>
 #include <string>
 
 #include "fb_launch.h"
+#include "fb_points.h"
 
 namespace fb {
 
@@ -26,148 +27,112 @@ constexpr int kBlock = 256;
 
 // ---------------------------------------------------------------------------
 // value offsets: (min + max)/2 over all values of a field, NaN if any value is NaN
-// (numpy's amin/amax propagate NaN), interpolation.py:209
+// (numpy's amin/amax propagate NaN), interpolation.py:209.  The smallest, the largest and the NaN
+// flag do not depend on the order of the reduction.
 
-// min, max and a NaN flag of v[k] for k = k0, k0 + kBlock, ... < k1, the loads of eight steps
-// issued before their first use (one thread's share of a workgroup's values)
-__device__ __forceinline__ void minmax_range(const double *__restrict__ v, int64_t k0, int64_t k1, double &mn,
-                                             double &mx, int &isn)
+// (min, max, NaN flag) of the workgroup's threads, valid in thread 0
+__device__ __forceinline__ void minmax_block(double &mn, double &mx, int &isn)
 {
-    constexpr int kUnroll = 8;
-    int64_t k = k0;
-    for (; k + (kUnroll - 1) * kBlock < k1; k += kUnroll * kBlock) {
-        double x[kUnroll];
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) x[u] = v[k + u * kBlock];
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (x[u] != x[u]) isn = 1;
-            mn = fmin(mn, x[u]);
-            mx = fmax(mx, x[u]);
-        }
+    __shared__ double smin[kBlock / 64], smax[kBlock / 64];
+    __shared__ int snan[kBlock / 64];
+    minmax_wave(mn, mx, isn);
+    if ((threadIdx.x & 63) == 0) {
+        smin[threadIdx.x >> 6] = mn;
+        smax[threadIdx.x >> 6] = mx;
+        snan[threadIdx.x >> 6] = isn;
     }
-    for (; k < k1; k += kBlock) {
-        const double x = v[k];
-        if (x != x) isn = 1;
-        mn = fmin(mn, x);
-        mx = fmax(mx, x);
-    }
-}
-
-__device__ __forceinline__ void offsets_block(const FieldDev *__restrict__ fields, const double *__restrict__ val,
-                                              double *__restrict__ offsets, int f)
-{
-    __shared__ double smin[kBlock], smax[kBlock];
-    __shared__ int snan;
-    const FieldDev &F = fields[f];
-    const int tid = threadIdx.x;
-    if (tid == 0) snan = 0;
-    double mn = INFINITY, mx = -INFINITY;
-    int isn = 0;
-    minmax_range(val + F.pt_off, tid, F.n, mn, mx, isn);
-    smin[tid] = mn;
-    smax[tid] = mx;
     __syncthreads();
-    if (isn) snan = 1;
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (tid < s) {
-            smin[tid] = fmin(smin[tid], smin[tid + s]);
-            smax[tid] = fmax(smax[tid], smax[tid + s]);
-        }
-        __syncthreads();
+    for (int w = 0; w < kBlock / 64; ++w) {
+        mn = fmin(mn, smin[w]);
+        mx = fmax(mx, smax[w]);
+        isn |= snan[w];
     }
-    if (tid == 0) offsets[f] = snan ? __builtin_nan("") : (smin[0] + smax[0]) / 2.0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_offsets(const FieldDev *__restrict__ fields,
                                                     const double *__restrict__ val, double *__restrict__ offsets)
 {
-    offsets_block(fields, val, offsets, blockIdx.x);
-}
-
-// The same over many workgroups per field (large fields): chunk c of field f (blockIdx.x,
-// blockIdx.y) reduces kOffChunk values to (min, max, NaN flag); k_offsets_final combines a
-// field's chunks.  min/max do not depend on the order, so the result equals k_offsets'.
-constexpr int kOffChunk = 8192;
-
-__global__ __launch_bounds__(kBlock) void k_offsets_part(const FieldDev *__restrict__ fields,
-                                                         const double *__restrict__ val, double *__restrict__ part)
-{
-    __shared__ double smin[kBlock], smax[kBlock];
-    __shared__ int snan;
-    const FieldDev &F = fields[blockIdx.y];
-    const int tid = threadIdx.x;
-    if (tid == 0) snan = 0;
-    const int64_t b0 = (int64_t)blockIdx.x * kOffChunk;
-    const int64_t b1 = min(F.n, b0 + kOffChunk);
+    const FieldDev &F = fields[blockIdx.x];
     double mn = INFINITY, mx = -INFINITY;
     int isn = 0;
-    minmax_range(val + F.pt_off, b0 + tid, b1, mn, mx, isn);
-    smin[tid] = mn;
-    smax[tid] = mx;
-    __syncthreads();
-    if (isn) snan = 1;
-    for (int st = kBlock / 2; st > 0; st >>= 1) {
-        if (tid < st) {
-            smin[tid] = fmin(smin[tid], smin[tid + st]);
-            smax[tid] = fmax(smax[tid], smax[tid + st]);
-        }
-        __syncthreads();
+    minmax_range(val + F.pt_off, threadIdx.x, F.n, kBlock, mn, mx, isn);
+    minmax_block(mn, mx, isn);
+    if (threadIdx.x == 0) offsets[blockIdx.x] = field_offset(mn, mx, isn);
+}
+
+// The same over many workgroups per field (large fields): workgroup f*nchunk + c reduces chunk c
+// (kOffChunk values) of field f to (min, max, NaN flag); offsets_final combines a field's chunks.
+constexpr int kOffChunk = 2048;     // values of a chunk
+constexpr int kOffSingle = 8192;    // fields of up to this many values: one workgroup each
+
+__device__ __forceinline__ void offsets_part(const FieldDev *__restrict__ fields, const double *__restrict__ val,
+                                             double *__restrict__ part, int64_t blk, int nchunk)
+{
+    const FieldDev &F = fields[blk / nchunk];
+    const int64_t b0 = (blk % nchunk) * kOffChunk;
+    double mn = INFINITY, mx = -INFINITY;
+    int isn = 0;
+    minmax_range(val + F.pt_off, b0 + threadIdx.x, min(F.n, b0 + kOffChunk), kBlock, mn, mx, isn);
+    minmax_block(mn, mx, isn);
+    if (threadIdx.x == 0) {
+        part[3 * blk] = mn;
+        part[3 * blk + 1] = mx;
+        part[3 * blk + 2] = isn ? 1.0 : 0.0;
     }
-    if (tid == 0) {
-        double *o = part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 3;
-        o[0] = smin[0];
-        o[1] = smax[0];
-        o[2] = snan ? 1.0 : 0.0;
+}
+
+// One wave per field.
+__device__ __forceinline__ void offsets_final(const double *__restrict__ part, int nfields, int nchunk,
+                                              double *__restrict__ offsets, int64_t blk)
+{
+    const int64_t f = blk * (kBlock / 64) + (threadIdx.x >> 6);
+    if (f >= nfields) return;
+    double mn = INFINITY, mx = -INFINITY;
+    int isn = 0;
+    for (int c = threadIdx.x & 63; c < nchunk; c += 64) {
+        const double *o = part + (f * nchunk + c) * 3;
+        mn = fmin(mn, o[0]);
+        mx = fmax(mx, o[1]);
+        if (o[2] != 0.0) isn = 1;
     }
+    minmax_wave(mn, mx, isn);
+    if ((threadIdx.x & 63) == 0) offsets[f] = field_offset(mn, mx, isn);
+}
+
+__global__ __launch_bounds__(kBlock) void k_offsets_part(const FieldDev *__restrict__ fields,
+                                                         const double *__restrict__ val, double *__restrict__ part,
+                                                         int nchunk)
+{
+    offsets_part(fields, val, part, blockIdx.x, nchunk);
 }
 
 __global__ __launch_bounds__(kBlock) void k_offsets_final(const double *__restrict__ part, int nfields, int nchunk,
                                                           double *__restrict__ offsets)
 {
-    const int f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nfields) return;
-    double mn = INFINITY, mx = -INFINITY;
-    bool isn = false;
-    for (int c = 0; c < nchunk; ++c) {
-        const double *o = part + ((int64_t)f * nchunk + c) * 3;
-        mn = fmin(mn, o[0]);
-        mx = fmax(mx, o[1]);
-        isn = isn || o[2] != 0.0;
+    offsets_final(part, nfields, nchunk, offsets, blockIdx.x);
+}
+
+// The first launch of the row-bucket sort stage: the offsets' chunks (the first noff workgroups) and
+// the zero fills, which do not depend on each other: the scan's counter `done`, the row counts and the
+// FP64 grids.
+constexpr int kZeroPer = 4;   // 16-byte stores of a thread
+
+__global__ __launch_bounds__(kBlock) void k_sort_begin(const FieldDev *__restrict__ fields,
+                                                       const double *__restrict__ val, double *__restrict__ part,
+                                                       int nchunk, int64_t noff, uint32_t *__restrict__ done,
+                                                       ZeroRange z0, ZeroRange z1, ZeroRange z2)
+{
+    if (blockIdx.x < noff) {
+        offsets_part(fields, val, part, blockIdx.x, nchunk);
+        return;
     }
-    offsets[f] = isn ? __builtin_nan("") : (mn + mx) / 2.0;
+    int64_t b = blockIdx.x - noff;
+    if (b == 0 && threadIdx.x == 0) *done = 0u;
+    if (zero_block<kBlock, kZeroPer>(z0, b) || zero_block<kBlock, kZeroPer>(z1, b)) return;
+    zero_block<kBlock, kZeroPer>(z2, b);
 }
 
 // ---------------------------------------------------------------------------
-// grid position of a point: xc = (p - x0)/step per axis, dropped when outside
-// [0, size-1) on any axis (interpolation.py:247-250).  NaN coordinates are
-// dropped as well (the reference's int(NaN) is undefined).
-
-struct PointPos {
-    int64_t i[3];
-    double w[3];
-};
-
-__device__ __forceinline__ bool point_pos(const FieldDev &F, const double *__restrict__ p, PointPos &pp)
-{
-    bool inside = true;
-    for (int m = 0; m < 3; ++m) {
-        pp.i[m] = 0;
-        pp.w[m] = 0.0;
-    }
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        if (m < F.dim) {
-            const double c = (p[m] - F.x0[m]) / F.step[m];
-            if (!(c >= 0.0) || c >= (double)(F.size[m] - 1)) inside = false;
-            const int64_t ci = inside ? (int64_t)c : 0;
-            pp.i[m] = ci;
-            pp.w[m] = c - (double)ci;
-        }
-    }
-    return inside;
-}
-
 // bilinear / trilinear corner weight of corner (bx, by, bz), formed left to right as
 // in the reference, e.g. (1.0-xw)*(1.0-yw) at interpolation.py:256
 __device__ __forceinline__ double corner_weight(int dim, const PointPos &pp, int64_t bx, int64_t by, int64_t bz)
@@ -178,74 +143,35 @@ __device__ __forceinline__ double corner_weight(int dim, const PointPos &pp, int
     return w;
 }
 
-// One (key, point) pair per point: the key is the point's base cell (the grid cell of its
-// lower corner), kInvalidKey for points the injection drops.  The corners of a point lie in
-// the base row (x-line) and the rows above it; counts per base row give, after the scan,
-// each row's range in the sorted pairs.
-__device__ __forceinline__ void point_keys_block(const FieldDev *__restrict__ fields,
-                                                 const int64_t *__restrict__ pt_prefix, int nfields, int64_t npoints,
-                                                 const double *__restrict__ pts, uint32_t *__restrict__ keys,
-                                                 uint32_t *__restrict__ vals, uint32_t *__restrict__ row_count,
-                                                 uint32_t *__restrict__ slot, uint32_t *__restrict__ rowg,
-                                                 PointRec *__restrict__ rec, int64_t blk)
+// A point's sort key is its base cell (the grid cell of its lower corner), kInvalidKey for points
+// the injection drops.  The corners of a point lie in the base row (x-line) and the rows above it;
+// counts per base row (integer atomics) give, after the scan, each row's range in the sorted list,
+// and slot is the point's position among its row's points as the atomics handed them out.  The
+// workgroups from nkb on take the fields' offsets from their chunks.
+__global__ __launch_bounds__(kBlock) void k_point_keys(const FieldDev *__restrict__ fields,
+                                                       const int64_t *__restrict__ pt_prefix, int nfields,
+                                                       int64_t npoints, const double *__restrict__ pts,
+                                                       uint32_t *__restrict__ keys, uint32_t *__restrict__ row_count,
+                                                       uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
+                                                       int64_t nkb, const double *__restrict__ part, int nchunk,
+                                                       double *__restrict__ offsets)
 {
-    // row_count (may be null): per-row point counts (integer atomics).  slot/rowg (row buckets): the point's
-    // position among its row's points as the atomics handed them out, and its global row
-    // (kInvalidKey outside the grid); vals (point indices) is then not written.
-    const int64_t i = blk * kBlock + threadIdx.x;
+    if (blockIdx.x >= nkb) {
+        offsets_final(part, nfields, nchunk, offsets, blockIdx.x - nkb);
+        return;
+    }
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= npoints) return;
-    const int f = find_seg(pt_prefix, nfields, i);
-    const FieldDev &F = fields[f];
+    const FieldDev &F = fields[find_seg(pt_prefix, nfields, i)];
     PointPos pp;
-    const bool inside = point_pos(F, pts + i * F.dim, pp);
-    if (!slot) vals[i] = (uint32_t)i;
-    if (!inside) {
+    if (!point_pos(F, pts + i * F.dim, pp)) {
         keys[i] = kInvalidKey;
-        if (rowg) rowg[i] = kInvalidKey;
         return;
     }
     const int64_t row = pp.i[2] * F.size[1] + pp.i[1];
     keys[i] = (uint32_t)(F.cell_off + row * F.size[0] + pp.i[0]);
     if (rec) rec[i] = PointRec{{pp.w[0], pp.w[1], pp.w[2]}, (int32_t)pp.i[0], 0};
-    if (row_count) {
-        const uint32_t sl = atomicAdd(&row_count[F.xline_off + row], 1u);
-        if (slot) {
-            slot[i] = sl;
-            rowg[i] = (uint32_t)(F.xline_off + row);
-        }
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_point_keys(const FieldDev *__restrict__ fields,
-                                                       const int64_t *__restrict__ pt_prefix, int nfields,
-                                                       int64_t npoints, const double *__restrict__ pts,
-                                                       uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
-                                                       uint32_t *__restrict__ row_count,
-                                                       uint32_t *__restrict__ slot, uint32_t *__restrict__ rowg,
-                                                       PointRec *__restrict__ rec)
-{
-    point_keys_block(fields, pt_prefix, nfields, npoints, pts, keys, vals, row_count, slot, rowg, rec, blockIdx.x);
-}
-
-// k_point_keys and k_offsets in one launch (they are independent): the first nkb workgroups
-// take the points, the next nfields the fields' offsets
-__global__ __launch_bounds__(kBlock) void k_point_keys_offsets(const FieldDev *__restrict__ fields,
-                                                               const int64_t *__restrict__ pt_prefix, int nfields,
-                                                               int64_t npoints, const double *__restrict__ pts,
-                                                               uint32_t *__restrict__ keys,
-                                                               uint32_t *__restrict__ vals,
-                                                               uint32_t *__restrict__ row_count,
-                                                               uint32_t *__restrict__ slot,
-                                                               uint32_t *__restrict__ rowg,
-                                                               PointRec *__restrict__ rec, int64_t nkb,
-                                                               const double *__restrict__ val,
-                                                               double *__restrict__ offsets)
-{
-    if ((int64_t)blockIdx.x < nkb)
-        point_keys_block(fields, pt_prefix, nfields, npoints, pts, keys, vals, row_count, slot, rowg, rec,
-                         blockIdx.x);
-    else
-        offsets_block(fields, val, offsets, (int)(blockIdx.x - nkb));
+    slot[i] = atomicAdd(&row_count[F.xline_off + row], 1u);
 }
 
 // k_point_keys for large point sets: each workgroup takes ppt*kBlock consecutive points and,
@@ -263,12 +189,17 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
                                                             const int64_t *__restrict__ pt_prefix, int nfields,
                                                             int64_t npoints, int ppt, int nbins,
                                                             const double *__restrict__ pts,
-                                                            uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
+                                                            uint32_t *__restrict__ keys,
                                                             uint32_t *__restrict__ row_count,
-                                                            uint32_t *__restrict__ slot, uint32_t *__restrict__ rowg,
-                                                            PointRec *__restrict__ rec)
+                                                            uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
+                                                            int64_t nkb, const double *__restrict__ part, int nchunk,
+                                                            double *__restrict__ offsets)
 {
     extern __shared__ uint32_t hist[];   // nbins row counters (dynamic LDS)
+    if (blockIdx.x >= nkb) {
+        offsets_final(part, nfields, nchunk, offsets, blockIdx.x - nkb);
+        return;
+    }
     __shared__ int64_t s_rbase;
     __shared__ int s_span;
     const int64_t p0 = (int64_t)blockIdx.x * ppt * kBlock;
@@ -347,10 +278,8 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
                     w[m] = cc - (double)q;
                 }
             }
-            if (!slot) vals[i] = (uint32_t)i;
             if (!inside) {
                 keys[i] = kInvalidKey;
-                if (rowg) rowg[i] = kInvalidKey;
                 continue;
             }
             const int64_t row = ci[2] * gsz[1] + ci[1];
@@ -361,11 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
                 rr[k] = (int)(grow - rbase);
                 lr[k] = atomicAdd(&hist[rr[k]], 1u);
             } else {
-                const uint32_t sl = atomicAdd(&row_count[grow], 1u);
-                if (slot) {
-                    slot[i] = sl;
-                    rowg[i] = (uint32_t)grow;
-                }
+                slot[i] = atomicAdd(&row_count[grow], 1u);
             }
         }
     }
@@ -376,14 +301,12 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
         const uint32_t c = hist[b];
         if (c) hist[b] = atomicAdd(&row_count[rbase + b], c);
     }
-    if (!slot) return;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kKeysMaxPpt; ++k) {
         if (rr[k] < 0) continue;
         const int64_t i = p0 + (int64_t)k * kBlock + threadIdx.x;
         slot[i] = hist[rr[k]] + lr[k];
-        rowg[i] = (uint32_t)(rbase + rr[k]);
     }
 }
 
@@ -424,22 +347,17 @@ __device__ __forceinline__ void line_streams(const FieldDev &F, int64_t line, bo
 
 // Each sorted entry's injection record, in list order: base column and row, point, field,
 // position within the base cell and value minus the offset, as point_pos forms them.  The
-// per-field sort (`local`) writes a field's in-grid points from its first point index on and
-// leaves the slots after them unused; the row-bucket sort packs all fields' entries by row.  Slots
-// past the list's last entry get row kInvalidKey.
+// row-bucket sort packs all fields' entries by row; slots past the list's last entry get row
+// kInvalidKey.  (k_field_sort writes its fields' records itself.)
 __global__ __launch_bounds__(kBlock) void k_inject_records(
     const FieldDev *__restrict__ fields, const int64_t *__restrict__ pt_prefix, int nfields, int64_t npoints,
-    int local, int64_t nxlines, const uint32_t *__restrict__ vals, const uint32_t *__restrict__ row_start,
+    int64_t nxlines, const uint32_t *__restrict__ vals, const uint32_t *__restrict__ row_start,
     const uint32_t *__restrict__ row_count, const double *__restrict__ pts, const double *__restrict__ val,
     const double *__restrict__ offsets, InjectRec *__restrict__ irec)
 {
     const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (e >= npoints) return;
-    int64_t last = nxlines - 1;   // the list's last row
-    if (local) {
-        const FieldDev &Fe = fields[find_seg(pt_prefix, nfields, e)];
-        last = Fe.xline_off + Fe.size[1] * Fe.size[2] - 1;   // the last row of the slot's field
-    }
+    const int64_t last = nxlines - 1;   // the list's last row
     if (e >= (int64_t)row_start[last] + row_count[last]) {
         irec[e].row = kInvalidKey;
         return;
@@ -1822,64 +1740,65 @@ int64_t offsets_part_elems(int nfields, int64_t max_n)
 int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
                    double *d_offsets, hipStream_t s)
 {
-    if (offsets_single_pass(max_n, d_part)) {
+    if (!d_part || max_n <= kOffSingle) {
         hipLaunchKernelGGL(k_offsets, dim3(nfields), dim3(kBlock), 0, s, d_fields, d_val, d_offsets);
     } else {
         const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
-        hipLaunchKernelGGL(k_offsets_part, dim3(nchunk, nfields), dim3(kBlock), 0, s, d_fields, d_val, d_part);
+        hipLaunchKernelGGL(k_offsets_part, dim3((unsigned)((int64_t)nchunk * nfields)), dim3(kBlock), 0, s, d_fields,
+                           d_val, d_part, nchunk);
         FB_HIP_CHECK(hipGetLastError());
-        hipLaunchKernelGGL(k_offsets_final, dim3((nfields + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
+        hipLaunchKernelGGL(k_offsets_final, dim3(nblocks((int64_t)nfields * 64)), dim3(kBlock), 0, s,
                            (const double *)d_part, nfields, nchunk, d_offsets);
     }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
 
-bool offsets_single_pass(int64_t max_n, const double *d_part) { return !d_part || max_n <= kOffChunk; }
-
-int launch_point_keys_offsets(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                              const double *d_pts, uint32_t *d_keys, uint32_t *d_vals, uint32_t *d_row_count,
-                              uint32_t *d_slot, uint32_t *d_rowg, const double *d_val, double *d_offsets,
-                              PointRec *d_rec, hipStream_t s)
+int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
+                      uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t s)
 {
-    if (nfields <= 0) return FB_OK;
-    const int64_t nkb = npoints > 0 ? nblocks(npoints) : 0;
-    hipLaunchKernelGGL(k_point_keys_offsets, dim3((unsigned)(nkb + nfields)), dim3(kBlock), 0, s, d_fields,
-                       d_pt_prefix, nfields, npoints, d_pts, d_keys, d_vals, d_row_count, d_slot, d_rowg, d_rec, nkb,
-                       d_val, d_offsets);
+    const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
+    const int64_t noff = (int64_t)nchunk * nfields;
+    int64_t nz = 0;
+    for (const ZeroRange &z : zero) nz += zero_blocks<kBlock, kZeroPer>(z);
+    hipLaunchKernelGGL(k_sort_begin, dim3((unsigned)(noff + std::max<int64_t>(nz, 1))), dim3(kBlock), 0, s, d_fields,
+                       d_val, d_part, nchunk, noff, d_done, zero[0], zero[1], zero[2]);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
 
-int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                      const double *d_pts, uint32_t *d_keys, uint32_t *d_vals, uint32_t *d_row_count,
-                      uint32_t *d_slot, uint32_t *d_rowg, int64_t max_rows, PointRec *d_rec, hipStream_t s)
+int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
+                      int64_t npoints, const double *d_pts, uint32_t *d_keys, uint32_t *d_row_count, uint32_t *d_slot,
+                      int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t s)
 {
-    if (npoints <= 0) return FB_OK;
+    if (nfields <= 0) return FB_OK;
+    const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
+    const unsigned nfin = nblocks((int64_t)nfields * 64);
     // points per thread: enough for each workgroup to see many points per row, while keeping
     // at least ~512 workgroups; small point sets, and fields with more rows than the LDS
     // counters (a workgroup of k_point_keys_hist over them would take one atomic per point, for
     // several points per thread), take one atomic per point and one point per thread
     const int64_t q = npoints / (512 * (int64_t)kBlock);
     const int64_t ppt = q < kKeysMaxPpt ? q : kKeysMaxPpt;
-    if (ppt >= 4 && d_row_count && max_rows <= kKeysBinsMax) {
+    if (ppt >= 4 && max_rows <= kKeysBinsMax) {
         // 64 KB of counters only where the fields need them (they halve the workgroups per CU;
         // fast_pass_init raised the kernel's dynamic-LDS limit)
         const int nbins = max_rows <= kKeysBins ? kKeysBins : kKeysBinsMax;
-        const int64_t per = ppt * kBlock;
-        hipLaunchKernelGGL(k_point_keys_hist, dim3((unsigned)((npoints + per - 1) / per)), dim3(kBlock),
-                           (size_t)nbins * 4, s, d_fields, d_pt_prefix, nfields, npoints, (int)ppt, nbins, d_pts,
-                           d_keys, d_vals, d_row_count, d_slot, d_rowg, d_rec);
+        const int64_t per = ppt * kBlock, nkb = (npoints + per - 1) / per;
+        hipLaunchKernelGGL(k_point_keys_hist, dim3((unsigned)(nkb + nfin)), dim3(kBlock), (size_t)nbins * 4, s,
+                           d_fields, d_pt_prefix, nfields, npoints, (int)ppt, nbins, d_pts, d_keys, d_row_count, d_slot,
+                           d_rec, nkb, d_part, nchunk, d_offsets);
     } else {
-        hipLaunchKernelGGL(k_point_keys, dim3(nblocks(npoints)), dim3(kBlock), 0, s, d_fields, d_pt_prefix, nfields,
-                           npoints, d_pts, d_keys, d_vals, d_row_count, d_slot, d_rowg, d_rec);
+        const int64_t nkb = npoints > 0 ? nblocks(npoints) : 0;
+        hipLaunchKernelGGL(k_point_keys, dim3((unsigned)(nkb + nfin)), dim3(kBlock), 0, s, d_fields, d_pt_prefix,
+                           nfields, npoints, d_pts, d_keys, d_row_count, d_slot, d_rec, nkb, d_part, nchunk, d_offsets);
     }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
 
 int launch_inject_records(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                          bool local, int64_t nxlines, const uint32_t *d_vals, const uint32_t *d_row_start,
+                          int64_t nxlines, const uint32_t *d_vals, const uint32_t *d_row_start,
                           const uint32_t *d_row_count, const double *d_pts, const double *d_val,
                           const double *d_offsets, InjectRec *d_irec, hipStream_t s)
 {
@@ -1889,7 +1808,7 @@ int launch_inject_records(const FieldDev *d_fields, const int64_t *d_pt_prefix, 
         return FB_ERR_INVALID_ARGUMENT;
     }
     hipLaunchKernelGGL(k_inject_records, dim3((unsigned)((npoints + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                       d_fields, d_pt_prefix, nfields, npoints, local ? 1 : 0, nxlines, d_vals, d_row_start,
+                       d_fields, d_pt_prefix, nfields, npoints, nxlines, d_vals, d_row_start,
                        d_row_count, d_pts, d_val, d_offsets, d_irec);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;

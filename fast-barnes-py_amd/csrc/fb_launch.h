@@ -7,16 +7,24 @@
 namespace fb {
 
 // fb_sort.hip
-int64_t scan_temp_elems(int64_t n);
-int scan_exclusive(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *tmp, hipStream_t stream);
-// per-field sort in LDS (fields of at most kLocalSortMax points): the sorted in-grid points
-// of field f from out_vals[pt_prefix[f]] on, in the same order as the row buckets; from the
-// per-row point counts d_row_count it writes the rows' starts d_row_start (the range of field
-// f begins at pt_prefix[f], so no scan over all rows is needed)
+// The whole sort stage of fields of at most kLocalSortMax points and kLocalRowsMax x-lines, one
+// workgroup each: the value offset (0 with `raw`), the rows' counts and starts (the range of field f
+// begins at pt_prefix[f]) and the in-grid points in the row buckets' order: the point list (d_out_vals)
+// with each point's PointRec (d_rec), or, with d_irec, the list of FP64 injection records, whose
+// unused slots get row kInvalidKey.  Further workgroups zero the ranges.
 int field_sort_init();
-int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int max_n,
-                      const uint32_t *d_keys, const uint32_t *d_row_count, uint32_t *d_row_start,
-                      uint32_t *d_out_vals, hipStream_t stream);
+int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int dim, int max_n,
+                      int max_rows, const double *d_pts, const double *d_val, bool raw, double *d_offsets,
+                      uint32_t *d_row_count, uint32_t *d_row_start, uint32_t *d_out_vals, PointRec *d_rec,
+                      InjectRec *d_irec, const ZeroRange (&zero)[2], hipStream_t stream);
+// fb_sort.hip -- row buckets for all other plans: the row starts from the row counts (scan_tiles(nrows)
+// words of d_tiles and the zeroed counter d_done), the in-grid points into their rows (d_comp), each
+// row sorted by (key, point index) into d_list, which may be d_keys' memory.
+int64_t scan_tiles(int64_t n);
+int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, const uint32_t *d_keys,
+                    const uint32_t *d_slot, int64_t npoints, uint32_t *d_row_start, const uint32_t *d_row_count,
+                    int64_t nrows, uint32_t *d_tiles, uint32_t *d_done, unsigned long long *d_comp, uint32_t *d_list,
+                    hipStream_t stream);
 
 // fb_kernels.hip -- injection front end
 // (min+max)/2 per field; with d_part (offsets_part_elems doubles) large fields are reduced
@@ -24,34 +32,21 @@ int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
 int64_t offsets_part_elems(int nfields, int64_t max_n);
 int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
                    double *d_offsets, hipStream_t stream);
-// one (base cell, point) pair per point and, unless d_row_count is NULL, per-base-row point
-// counts (row = x-line index) by integer atomics; with d_slot/d_rowg (row buckets) each point's
-// slot in its row and its row instead of the point indices.  max_rows: the most x-lines of any
-// field.  d_rec (may be NULL): each in-grid point's PointRec, for the FP32C injection
-int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                      const double *d_pts, uint32_t *d_keys, uint32_t *d_vals, uint32_t *d_row_count,
-                      uint32_t *d_slot, uint32_t *d_rowg, int64_t max_rows, PointRec *d_rec, hipStream_t stream);
-// launch_point_keys and, when the offsets take one workgroup per field (offsets_single_pass),
-// launch_offsets in one launch
-bool offsets_single_pass(int64_t max_n, const double *d_part);
-int launch_point_keys_offsets(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                              const double *d_pts, uint32_t *d_keys, uint32_t *d_vals, uint32_t *d_row_count,
-                              uint32_t *d_slot, uint32_t *d_rowg, const double *d_val, double *d_offsets,
-                              PointRec *d_rec, hipStream_t stream);
-// fb_sort.hip -- row buckets for fields of more than kLocalSortMax points: scatter the in-grid
-// points into their rows (d_row_start from the scan of the counts), then sort each row by
-// (key, point index); d_svals/d_skeys receive the sorted list, d_tkeys/d_tvals are scratch for
-// rows of more than kLocalSortMax points; d_big_list holds 2*nrows entries and d_big_count 2
-// counters, which must be zero
-int row_bucket_sort(const uint32_t *d_keys, const uint32_t *d_slot, const uint32_t *d_rowg, int64_t npoints,
-                    const uint32_t *d_row_start, const uint32_t *d_row_count, int64_t nrows, uint32_t *d_skeys,
-                    uint32_t *d_svals, uint32_t *d_big_list, uint32_t *d_big_count, uint32_t *d_tkeys,
-                    uint32_t *d_tvals, hipStream_t stream);
+// The row buckets' first two launches.  launch_sort_begin: the offsets' chunks (d_part), *d_done = 0
+// and the ranges zeroed.  launch_point_keys: the offsets from the chunks; each point's base cell,
+// its base row's count (row = x-line index, integer atomics on zeroed counts) and its slot there.
+// max_rows: the most x-lines of any field.  d_rec (may be NULL): each in-grid point's PointRec, for
+// the FP32C injection
+int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
+                      uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t stream);
+int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
+                      int64_t npoints, const double *d_pts, uint32_t *d_keys, uint32_t *d_row_count, uint32_t *d_slot,
+                      int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t stream);
 
 // fb_kernels.hip -- FP64 path with the reference's operation order
-// Each sorted entry's FP64 injection record (local: the per-field sort's layout).
+// Each sorted entry's FP64 injection record (row buckets).
 int launch_inject_records(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
-                          bool local, int64_t nxlines, const uint32_t *d_vals, const uint32_t *d_row_start,
+                          int64_t nxlines, const uint32_t *d_vals, const uint32_t *d_row_start,
                           const uint32_t *d_row_count, const double *d_pts, const double *d_val,
                           const double *d_offsets, InjectRec *d_irec, hipStream_t stream);
 // The injection sums of every cell that receives any, in point order; the grids must be cleared

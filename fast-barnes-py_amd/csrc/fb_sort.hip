@@ -1,66 +1,93 @@
-// fb_sort.hip -- exclusive scan, the per-field sort in LDS (fields of at most kLocalSortMax
-// points) and the row-bucket sort (larger fields).
+// fb_sort.hip -- the sort stage: fields of few points in one launch (k_field_sort), all others by
+// row buckets (scan of the row counts, scatter into the rows, row sorts).
 //
 // Used to order the injection's points by base cell while keeping, inside a cell, the point
 // order of the input (the order in which the reference's _inject_data_*d loop adds them,
 // interpolation.py:246-270): both sorts order the composite (cell key, point index), so the
 // result does not depend on timing.
+#include <algorithm>
 #include <mutex>
 
 #include "fb_internal.h"
 #include "fb_launch.h"
+#include "fb_points.h"
 
 namespace fb {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kItems = 16;
-constexpr int kTile = kThreads * kItems;   // 4096 elements per workgroup of the multi-level scan
+constexpr int kItems = 4;
+constexpr int kTile = kThreads * kItems;   // 1024 elements per workgroup of the scan
 constexpr int kLocalSortThreads = 1024;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// ---- scan ----------------------------------------------------------------
-
-__global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restrict__ in,
-                                                         uint32_t *__restrict__ out,
-                                                         uint32_t *__restrict__ tile_sums, int64_t n)
+// Sum of v over the workgroup's earlier threads; total: over all of them.  wsum: one word per wave
+// (nobody may still read it).
+__device__ __forceinline__ uint32_t block_before(uint32_t v, uint32_t *wsum, uint32_t &total)
 {
-    __shared__ uint32_t s_tot[kThreads];
-    const int tid = threadIdx.x;
-    const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)tid * kItems;
-    uint32_t v[kItems];
-    uint32_t sum = 0;
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-        const int64_t idx = base + i;
-        v[i] = idx < n ? in[idx] : 0u;
-        sum += v[i];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    uint32_t inc = v;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
     }
-    s_tot[tid] = sum;
+    if (lane == 63) wsum[wv] = inc;
     __syncthreads();
-    for (int off = 1; off < kThreads; off <<= 1) {
-        const uint32_t t = tid >= off ? s_tot[tid - off] : 0u;
-        __syncthreads();
-        s_tot[tid] += t;
-        __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+    for (int w = 0; w < nw; ++w) {
+        const uint32_t x = wsum[w];
+        before += w < wv ? x : 0u;
+        total += x;
     }
-    uint32_t run = tid ? s_tot[tid - 1] : 0u;
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) {
-        const int64_t idx = base + i;
-        if (idx < n) out[idx] = run;
-        run += v[i];
-    }
-    if (tid == kThreads - 1 && tile_sums) tile_sums[blockIdx.x] = s_tot[kThreads - 1];
+    return before + inc - v;
 }
 
-__global__ __launch_bounds__(kThreads) void k_scan_add(uint32_t *__restrict__ out,
-                                                       const uint32_t *__restrict__ tile_offs, int64_t n)
+// ---- scan ----------------------------------------------------------------
+
+// out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of all tiles
+// before tile t, formed by the workgroup that ends last (no workgroup waits for another).
+__global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
+                                                         int64_t n, uint32_t *__restrict__ tiles,
+                                                         uint32_t *__restrict__ done)
 {
-    const int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (idx < n) out[idx] += tile_offs[idx / kTile];
+    __shared__ uint32_t wsum[kThreads / 64];
+    __shared__ uint32_t last;
+    const int tid = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)tid * kItems;
+    uint32_t v[kItems] = {}, sum = 0, total;
+    if (base + kItems <= n) {
+        const uint4 x = *reinterpret_cast<const uint4 *>(in + base);
+        v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) v[i] = base + i < n ? in[base + i] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) sum += v[i];
+    uint32_t run = block_before(sum, wsum, total);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        if (base + i < n) out[base + i] = run;
+        run += v[i];
+    }
+    if (tid == 0) {
+        __hip_atomic_store(&tiles[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    uint32_t carry = 0;
+    for (int64_t t0 = 0; t0 < gridDim.x; t0 += kThreads) {
+        const int64_t t = t0 + tid;
+        const uint32_t x = t < gridDim.x ? __hip_atomic_load(&tiles[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+        const uint32_t before = block_before(x, wsum, total);
+        if (t < gridDim.x) tiles[t] = carry + before;
+        carry += total;
+        __syncthreads();   // wsum is rewritten
+    }
 }
 
 // Bitonic network over sk[0, np2) (np2 a power of two) in LDS by the whole workgroup, ascending.
@@ -92,194 +119,274 @@ __device__ __forceinline__ void block_bitonic(unsigned long long *sk, int np2)
     __syncthreads();
 }
 
-// One workgroup per field: the field's points inside the grid written in (cell key, point
-// index) order (equal keys stay in point order, as in the row-bucket sort) into the field's
-// range of the list, which begins at the field's first point index (pt_prefix[f]; the range
-// holds n slots, of which the in-grid points fill the first).  Keys order by row first (key =
-// cell_off + row*W + x), and k_point_keys has counted each row's points: the workgroup scans the
-// field's row counts into the rows' starts (written to row_start, absolute).  When the field
-// has at most kFieldRows rows and none holds more than kRankMax points, every point goes to
-// its row's start plus its rank among the row's points: the points are dropped into their
-// rows' ranges in LDS (atomic cursors, any order), then each counts the row's entries below
-// its own composite.  Otherwise a bitonic network sorts the 64-bit composites in LDS.  Both
-// give the same order.  Fields of at most kLocalSortMax points.
-constexpr int kFieldRows = 4096;                                    // LDS row starts and cursors
-constexpr int kRankMax = 64;                                        // largest row placed by rank
+// ---- fields of at most kLocalSortMax points and kLocalRowsMax rows ----------------------------
+// One workgroup per field takes its whole sort stage: the value offset; each point's base cell; the
+// rows' counts and starts (absolute: a field's list begins at its first point index, pt_prefix[f], and
+// its in-grid points fill the first of its slots); and the points in (cell key, point index) order.
+// The points are counted in LDS by buckets, 2^ls column ranges of each row, and dropped into the
+// buckets' ranges; when no bucket holds more than kRankMax points each point's place is its bucket's
+// start plus the number of the bucket's entries below its own.  Otherwise a bitonic network sorts the
+// 64-bit composites in LDS.  Both give the same order.
+//
+// EXACT: the list is written as FP64 injection records (irec), else as point indices (out_vals),
+// with each point's position in rec.  The workgroups after the fields' zero the FP64 grids meanwhile.
+//
+// Bound by latency, one workgroup's chain of loads, divisions and LDS steps.  kBuckets buckets, as
+// many as there may be points, keep the last step short: with one bucket per row (12 to 40 points) it
+// took 6 us more.  5001 points on 601x299: zero fill, keys with the offset and sort took 1.9 + 5.5 +
+// 15.6 us in launches of their own, this takes 14.8.
+struct FieldSortArgs {
+    const FieldDev *fields;
+    const int64_t *pt_prefix;
+    const double *pts, *val;
+    double *offsets;
+    uint32_t *row_count, *row_start, *out_vals;
+    PointRec *rec;
+    InjectRec *irec;
+    ZeroRange zero[2];
+    int nfields, np2, raw;   // np2: the LDS composites; raw: offset 0
+};
+
+constexpr int kBuckets = 8192;                                      // at least 2 * kLocalRowsMax
+constexpr int kRankMax = 64;                                        // largest bucket placed by rank
 constexpr int kSortPerThread = kLocalSortMax / kLocalSortThreads;   // points per thread
+constexpr int kBucketsPerThread = kBuckets / kLocalSortThreads;
 constexpr int kSortWaves = kLocalSortThreads / 64;
+constexpr int kSortZeroPer = 8;   // 16-byte stores of a zeroing thread
+constexpr int kRankStep = 4;      // LDS reads in flight of a rank; sk has as many entries to spare
 
-__global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(const FieldDev *__restrict__ fields,
-                                                                  const int64_t *__restrict__ pt_prefix,
-                                                                  const uint32_t *__restrict__ keys,
-                                                                  const uint32_t *__restrict__ row_count,
-                                                                  uint32_t *__restrict__ row_start,
-                                                                  uint32_t *__restrict__ out_vals)
+template <int DIM, bool EXACT>
+__global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs A)
 {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ uint32_t cur[kFieldRows];
-    __shared__ uint32_t rst[kFieldRows];
-    __shared__ uint32_t wsum[kSortWaves];
-    unsigned long long *sk = reinterpret_cast<unsigned long long *>(smem);
-    const int f = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wv = tid >> 6;
-    const FieldDev &F = fields[f];
-    const int64_t p0 = pt_prefix[f];
-    const int n = (int)(pt_prefix[f + 1] - p0);
-    const int64_t r0 = F.xline_off;
-    const int64_t nr = F.size[1] * F.size[2];   // x-lines (rows) of the field
-    const uint32_t dst = (uint32_t)p0;
-
-    // exclusive scan of the row counts (chunks of one row per thread) and the largest row
-    uint32_t carry = 0, m = 0;
-    for (int64_t c0 = 0; c0 < nr; c0 += kLocalSortThreads) {
-        const int64_t r = c0 + tid;
-        const uint32_t v = r < nr ? row_count[r0 + r] : 0u;
-        m = max(m, v);
-        uint32_t inc = v;
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t o = __shfl_up(inc, d);
-            if (lane >= d) inc += o;
-        }
-        if (lane == 63) wsum[wv] = inc;
-        __syncthreads();
-        uint32_t before = 0, total = 0;
-#pragma unroll
-        for (int w = 0; w < kSortWaves; ++w) {
-            const uint32_t x = wsum[w];
-            before += w < wv ? x : 0u;
-            total += x;
-        }
-        const uint32_t ex = carry + before + inc - v;
-        if (r < nr) {
-            row_start[r0 + r] = dst + ex;
-            if (r < kFieldRows) rst[r] = ex;
-        }
-        carry += total;
-        __syncthreads();   // wsum is rewritten by the next chunk
+    extern __shared__ __align__(16) unsigned char smem[];   // composites
+    __shared__ __align__(16) uint32_t start[kBuckets + 4];  // the buckets' counts, then their starts
+    __shared__ uint32_t wsum[kSortWaves], wmax[kSortWaves];
+    __shared__ double dmin[kSortWaves], dmax[kSortWaves];
+    __shared__ int dnan[kSortWaves];
+    if ((int64_t)blockIdx.x >= A.nfields) {
+        int64_t b = (int64_t)blockIdx.x - A.nfields;
+        if (!zero_block<kLocalSortThreads, kSortZeroPer>(A.zero[0], b))
+            zero_block<kLocalSortThreads, kSortZeroPer>(A.zero[1], b);
+        return;
     }
-    for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d));
-    if (lane == 0) wsum[wv] = m;
-    __syncthreads();
-    uint32_t mx = 0;
-#pragma unroll
-    for (int w = 0; w < kSortWaves; ++w) mx = max(mx, wsum[w]);
+    const int f = blockIdx.x, tid = threadIdx.x, wv = tid >> 6;
+    FieldDev F = A.fields[f];   // by value: the stores below cannot change it
+    F.dim = DIM;
+    const int64_t p0 = A.pt_prefix[f];
+    const int n = (int)(A.pt_prefix[f + 1] - p0);
+    const int nr = (int)(F.size[1] * F.size[2]);   // x-lines (rows) of the field
+    const uint32_t dst = (uint32_t)p0;
+    unsigned long long *const sk = reinterpret_cast<unsigned long long *>(smem);
+    // bucket = row << ls | column range; the range ascends with the column
+    int ls = 0;
+    while (nr << (ls + 1) <= kBuckets) ++ls;
+    const float bscale = (float)(1 << ls) / (float)F.size[0];
 
-    if (nr <= kFieldRows && mx <= (uint32_t)kRankMax) {
-        for (int r = tid; r < nr; r += kLocalSortThreads) cur[r] = 0u;
-        __syncthreads();
-        const uint32_t cbase = (uint32_t)F.cell_off, W = (uint32_t)F.size[0];
-        unsigned long long ev[kSortPerThread];
-        uint32_t rs[kSortPerThread], rc[kSortPerThread];
+    uint4 *const quads = reinterpret_cast<uint4 *>(start);
+    double mn = INFINITY, mx = -INFINITY;
+    int isn = 0;
+    int xi[kSortPerThread];            // base column, -1 outside the grid
+    uint32_t bs[kSortPerThread];       // bucket, slot in it << 16
+    double v[kSortPerThread], w[EXACT ? kSortPerThread : 1][DIM];
+    // coordinates and values of kGroup points in flight together (as many as there are registers for)
+    constexpr int kGroup = EXACT && DIM >= 3 ? kSortPerThread / 4 : kSortPerThread;
 #pragma unroll
-        for (int k = 0; k < kSortPerThread; ++k) {
-            const int i = tid + k * kLocalSortThreads;
-            rc[k] = 0u;
-            rs[k] = 0u;
-            ev[k] = 0ull;
+    for (int g = 0; g < kSortPerThread; g += kGroup) {
+        double c[kGroup][DIM];
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+            const int i = tid + (g + u) * kLocalSortThreads;
             if (i < n) {
-                const uint32_t key = keys[p0 + i];
-                if (key != kInvalidKey) {
-                    const uint32_t r = (key - cbase) / W;
-                    rs[k] = rst[r];   // the row's range in the field's list
-                    rc[k] = row_count[r0 + r];
-                    ev[k] = ((unsigned long long)key << 32) | (unsigned long long)(uint32_t)(p0 + i);
-                    sk[rs[k] + atomicAdd(&cur[r], 1u)] = ev[k];
+                v[g + u] = A.val[p0 + i];
+#pragma unroll
+                for (int m = 0; m < DIM; ++m) c[u][m] = A.pts[(p0 + i) * DIM + m];
+            }
+        }
+        if (g == 0) {
+#pragma unroll
+            for (int q = 0; q < kBucketsPerThread / 4; ++q)
+                quads[tid + q * kLocalSortThreads] = make_uint4(0u, 0u, 0u, 0u);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+            const int k = g + u, i = tid + k * kLocalSortThreads;
+            xi[k] = -1;
+            if (i < n) {
+                if (v[k] != v[k]) isn = 1;
+                mn = fmin(mn, v[k]);
+                mx = fmax(mx, v[k]);
+                PointPos pp;
+                if (point_pos(F, c[u], pp)) {
+                    const int row = (int)(DIM >= 3 ? pp.i[2] * F.size[1] + pp.i[1] : pp.i[1]);
+                    xi[k] = (int)pp.i[0];
+                    const uint32_t b = (uint32_t)row << ls | min((uint32_t)((float)xi[k] * bscale), (1u << ls) - 1u);
+                    bs[k] = b | atomicAdd(&start[b], 1u) << 16;
+                    if constexpr (EXACT) {
+#pragma unroll
+                        for (int m = 0; m < DIM; ++m) w[k][m] = pp.w[m];
+                    } else {
+                        A.rec[p0 + i] = PointRec{{pp.w[0], pp.w[1], pp.w[2]}, xi[k], 0};
+                    }
                 }
             }
         }
+    }
+    minmax_wave(mn, mx, isn);
+    if ((tid & 63) == 0) {
+        dmin[wv] = mn;
+        dmax[wv] = mx;
+        dnan[wv] = isn;
+    }
+    __syncthreads();
+
+    // the buckets' starts (consecutive buckets per thread) and the largest bucket
+    uint32_t rc[kBucketsPerThread], sum = 0, big = 0, total;
+#pragma unroll
+    for (int q = 0; q < kBucketsPerThread; q += 4) {
+        const uint4 x = quads[tid * (kBucketsPerThread / 4) + q / 4];
+        rc[q] = x.x, rc[q + 1] = x.y, rc[q + 2] = x.z, rc[q + 3] = x.w;
+    }
+#pragma unroll
+    for (int q = 0; q < kBucketsPerThread; ++q) {
+        sum += rc[q];
+        big = max(big, rc[q]);
+    }
+    for (int d = 32; d >= 1; d >>= 1) big = max(big, (uint32_t)__shfl_xor((int)big, d));
+    if ((tid & 63) == 0) wmax[wv] = big;
+    uint32_t run = block_before(sum, wsum, total);
+#pragma unroll
+    for (int q = 0; q < kBucketsPerThread; ++q) {
+        const uint32_t x = rc[q];
+        rc[q] = run;
+        run += x;
+    }
+#pragma unroll
+    for (int q = 0; q < kBucketsPerThread; q += 4)
+        quads[tid * (kBucketsPerThread / 4) + q / 4] = make_uint4(rc[q], rc[q + 1], rc[q + 2], rc[q + 3]);
+    if (tid == kLocalSortThreads - 1) start[kBuckets] = run;
+#pragma unroll
+    for (int q = 0; q < kSortWaves; ++q) {
+        big = max(big, wmax[q]);
+        mn = fmin(mn, dmin[q]);
+        mx = fmax(mx, dmax[q]);
+        isn |= dnan[q];
+    }
+    const double off = A.raw ? 0.0 : field_offset(mn, mx, isn);
+    if (tid == 0) A.offsets[f] = off;
+    __syncthreads();
+    for (int r = tid; r < nr; r += kLocalSortThreads) {
+        const uint32_t s0 = start[r << ls];
+        A.row_start[F.xline_off + r] = dst + s0;
+        A.row_count[F.xline_off + r] = start[(r + 1) << ls] - s0;
+    }
+    if constexpr (EXACT)
+        for (int i = (int)total + tid; i < n; i += kLocalSortThreads) A.irec[dst + i].row = kInvalidKey;
+
+    if (big <= (uint32_t)kRankMax) {
+#pragma unroll
+        for (int k = 0; k < kSortPerThread; ++k)
+            if (xi[k] >= 0)
+                sk[start[bs[k] & 0xffffu] + (bs[k] >> 16)] =
+                    ((unsigned long long)(uint32_t)xi[k] << 32) | (uint32_t)(p0 + tid + k * kLocalSortThreads);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < kSortPerThread; ++k) {
-            if (rc[k] == 0u) continue;
-            uint32_t rank = 0;
-            for (uint32_t j = 0; j < rc[k]; ++j) rank += sk[rs[k] + j] < ev[k] ? 1u : 0u;
-            out_vals[dst + rs[k] + rank] = (uint32_t)ev[k];
+            if (xi[k] < 0) continue;
+            const uint32_t p = (uint32_t)(p0 + tid + k * kLocalSortThreads);
+            const unsigned long long e = ((unsigned long long)(uint32_t)xi[k] << 32) | p;
+            const uint32_t b = bs[k] & 0xffffu, s0 = start[b], s1 = start[b + 1];
+            uint32_t at = s0;
+            for (uint32_t j = s0; j < s1; j += kRankStep) {
+                unsigned long long x[kRankStep];
+#pragma unroll
+                for (int u = 0; u < kRankStep; ++u) x[u] = sk[j + u];
+#pragma unroll
+                for (int u = 0; u < kRankStep; ++u) at += j + u < s1 && x[u] < e ? 1u : 0u;
+            }
+            if constexpr (EXACT) {
+                // (three axes leave no registers for the values)
+                InjectRec R{xi[k], p, (uint32_t)(F.xline_off + (b >> ls)), f, 0.0, 0.0, 0.0,
+                            (DIM >= 3 ? A.val[p] : v[k]) - off};
+                R.wx = w[k][0];
+                if constexpr (DIM >= 2) R.wy = w[k][1];
+                if constexpr (DIM >= 3) R.wz = w[k][2];
+                A.irec[dst + at] = R;
+            } else {
+                A.out_vals[dst + at] = p;
+            }
         }
         return;
     }
 
-    int np2 = 1;
-    while (np2 < n) np2 <<= 1;
-    for (int i = tid; i < np2; i += kLocalSortThreads)
-        sk[i] = i < n ? ((unsigned long long)keys[p0 + i] << 32) | (unsigned long long)(uint32_t)(p0 + i) : ~0ull;
+    const uint32_t W = (uint32_t)F.size[0];
+    for (int i = n + tid; i < A.np2; i += kLocalSortThreads) sk[i] = ~0ull;
+#pragma unroll
+    for (int k = 0; k < kSortPerThread; ++k) {
+        const int i = tid + k * kLocalSortThreads;
+        if (i < n)
+            sk[i] = xi[k] < 0 ? ~0ull
+                              : ((unsigned long long)(((bs[k] & 0xffffu) >> ls) * W + (uint32_t)xi[k]) << 32) |
+                                    (uint32_t)(p0 + i);
+    }
     __syncthreads();
-    block_bitonic(sk, np2);
-    for (int i = tid; i < n; i += kLocalSortThreads) {
-        const unsigned long long e = sk[i];
-        if ((uint32_t)(e >> 32) != kInvalidKey) out_vals[dst + i] = (uint32_t)e;
+    block_bitonic(sk, A.np2);
+    for (int i = tid; i < (int)total; i += kLocalSortThreads) {
+        const uint32_t p = (uint32_t)sk[i];
+        if constexpr (EXACT) {
+            PointPos pp;
+            point_pos(F, A.pts + (int64_t)p * DIM, pp);
+            A.irec[dst + i] = InjectRec{(int)pp.i[0], p, (uint32_t)(F.xline_off + pp.i[2] * F.size[1] + pp.i[1]), f,
+                                        pp.w[0], pp.w[1], pp.w[2], A.val[p] - off};
+        } else {
+            A.out_vals[dst + i] = p;
+        }
     }
 }
 
-// ---- row buckets (fields of more than kLocalSortMax points) ------------------
+// ---- row buckets (all other plans) ------------------------------------------------------------
 // The order of a stable sort of the (cell key, point index) pairs: every in-grid point
 // has a slot in its base row (k_point_keys' atomic count), the rows start at the exclusive scan
 // of the counts, and each row's entries are then sorted by the composite (key, point index).
 
-constexpr int kRowSmall = 16;           // rows of at most this many entries: one thread, in registers
-constexpr int kRowWave = 1024;          // rows of at most this many entries: one wave, in LDS ...
-constexpr int kRankWave = 256;          // ... by rank up to this many, by a bitonic network above
-constexpr int kRowSortThreads = 256;    // workgroup of the wave kernel (4 rows at a time) and of larger rows
+constexpr int kRowSmall = 16;      // rows of at most this many entries: one thread, in registers
+constexpr int kRowWave = 512;      // rows of at most this many entries: one wave, in LDS ...
+constexpr int kRankWave = 256;     // ... by rank up to this many, by a bitonic network above
+constexpr int kRowThreads = 1024;  // workgroup of the row sorts: 16 waves share kLocalSortMax composites
+constexpr int kRowGrid = 512;      // ... and their number, at most
 
-__device__ __forceinline__ unsigned long long row_entry(const uint32_t *keys, const uint32_t *vals, uint32_t i)
-{
-    return ((unsigned long long)keys[i] << 32) | (unsigned long long)vals[i];
-}
-
-__global__ __launch_bounds__(kThreads) void k_row_scatter(int64_t n, const uint32_t *__restrict__ keys,
+__global__ __launch_bounds__(kThreads) void k_row_scatter(const FieldDev *__restrict__ fields,
+                                                          const int64_t *__restrict__ pt_prefix, int nfields, int64_t n,
+                                                          const uint32_t *__restrict__ keys,
                                                           const uint32_t *__restrict__ slot,
-                                                          const uint32_t *__restrict__ rowg,
                                                           const uint32_t *__restrict__ row_start,
-                                                          uint32_t *__restrict__ skeys, uint32_t *__restrict__ svals)
+                                                          const uint32_t *__restrict__ tiles,
+                                                          unsigned long long *__restrict__ comp)
 {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    const uint32_t r = rowg[i];
-    if (r == kInvalidKey) return;   // outside its grid
-    const uint32_t dst = row_start[r] + slot[i];
-    skeys[dst] = keys[i];
-    svals[dst] = (uint32_t)i;
+    const uint32_t key = keys[i], sl = slot[i];
+    if (key == kInvalidKey) return;   // outside its grid
+    const FieldDev &F = fields[find_seg(pt_prefix, nfields, i)];
+    const int64_t r = F.xline_off + (key - (uint32_t)F.cell_off) / (uint32_t)F.size[0];
+    comp[row_start[r] + tiles[r / kTile] + sl] = ((unsigned long long)key << 32) | (unsigned long long)(uint32_t)i;
 }
 
-// One thread per row: rows of 2..kRowSmall entries sorted by a bitonic network in registers
-// (padded with the largest composite); rows of up to kRowWave entries are appended to
-// lists[0] (count counts[0]), larger ones to lists[1] (counts[1]).
-__global__ __launch_bounds__(kThreads) void k_row_sort_small(int64_t nrows, const uint32_t *__restrict__ row_start,
-                                                             const uint32_t *__restrict__ row_count,
-                                                             uint32_t *__restrict__ skeys,
-                                                             uint32_t *__restrict__ svals,
-                                                             uint32_t *__restrict__ lists,
-                                                             uint32_t *__restrict__ counts)
+// One thread sorts a row of n <= M entries by a bitonic network in registers (padded with the
+// largest composite).
+template <int M>
+__device__ __forceinline__ void small_row(const unsigned long long *__restrict__ comp, uint32_t *__restrict__ list,
+                                          uint32_t s0, uint32_t n)
 {
-    const int64_t r = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const uint32_t n = r < nrows ? row_count[r] : 0;
-    // list appends aggregated per wave: one atomic per wave and list (a single counter taking
-    // one atomic per row serialises when most rows are large)
-    const int lane = threadIdx.x & 63;
-    const unsigned long long below = (1ull << lane) - 1ull;
+    unsigned long long e[M];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const bool mine = c == 0 ? (n > (uint32_t)kRowSmall && n <= (uint32_t)kRowWave) : n > (uint32_t)kRowWave;
-        const unsigned long long m = __ballot(mine);
-        if (m) {
-            const int leader = __ffsll((long long)m) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&counts[c], (uint32_t)__popcll(m));
-            base = __shfl(base, leader);
-            if (mine) lists[c * nrows + base + (uint32_t)__popcll(m & below)] = (uint32_t)r;
-        }
-    }
-    if (n <= 1 || n > (uint32_t)kRowSmall) return;
-    const uint32_t s0 = row_start[r];
-    unsigned long long e[kRowSmall];
+    for (int q = 0; q < M; ++q) e[q] = (uint32_t)q < n ? comp[s0 + q] : ~0ull;
 #pragma unroll
-    for (int q = 0; q < kRowSmall; ++q) e[q] = (uint32_t)q < n ? row_entry(skeys, svals, s0 + q) : ~0ull;
-#pragma unroll
-    for (int k = 2; k <= kRowSmall; k <<= 1)
+    for (int k = 2; k <= M; k <<= 1)
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1)
 #pragma unroll
-            for (int i = 0; i < kRowSmall; ++i) {
+            for (int i = 0; i < M; ++i) {
                 const int l = i ^ j;
                 if (l > i) {
                     const bool up = (i & k) == 0;
@@ -291,11 +398,8 @@ __global__ __launch_bounds__(kThreads) void k_row_sort_small(int64_t nrows, cons
                 }
             }
 #pragma unroll
-    for (int q = 0; q < kRowSmall; ++q)
-        if ((uint32_t)q < n) {
-            skeys[s0 + q] = (uint32_t)(e[q] >> 32);
-            svals[s0 + q] = (uint32_t)e[q];
-        }
+    for (int q = 0; q < M; ++q)
+        if ((uint32_t)q < n) list[s0 + q] = (uint32_t)e[q];
 }
 
 // One wave sorts the row of n <= 64*NU entries at s0 by rank: each entry's slot is the number of
@@ -304,21 +408,22 @@ __global__ __launch_bounds__(kThreads) void k_row_sort_small(int64_t nrows, cons
 // is padded with ~0, which no composite exceeds).  NU = ceil(n/64) keeps the compares to the
 // registers that hold entries.
 template <int NU>
-__device__ __forceinline__ void rank_row(uint32_t *__restrict__ skeys, uint32_t *__restrict__ svals, uint32_t s0,
-                                         uint32_t n, unsigned long long *__restrict__ sk, int lane)
+__device__ __forceinline__ void rank_row(const unsigned long long *__restrict__ comp, uint32_t *__restrict__ list,
+                                         uint32_t s0, uint32_t n, unsigned long long *__restrict__ sk, int lane)
 {
     unsigned long long e[NU];
     uint32_t rk[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
         const uint32_t i = lane + 64 * u;
-        e[u] = i < n ? row_entry(skeys, svals, s0 + i) : ~0ull;
+        e[u] = i < n ? comp[s0 + i] : ~0ull;
         if (i < n) sk[i] = e[u];
         rk[u] = 0u;
     }
     if (lane == 0 && (n & 1u)) sk[n] = ~0ull;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const ulonglong2 *sk2 = reinterpret_cast<const ulonglong2 *>(sk);
+#pragma unroll 4
     for (uint32_t j = 0; j < (n + 1) >> 1; ++j) {
         const ulonglong2 x = sk2[j];
 #pragma unroll
@@ -326,176 +431,134 @@ __device__ __forceinline__ void rank_row(uint32_t *__restrict__ skeys, uint32_t 
     }
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-        if (lane + 64 * u < (int)n) {
-            skeys[s0 + rk[u]] = (uint32_t)(e[u] >> 32);
-            svals[s0 + rk[u]] = (uint32_t)e[u];
-        }
+        if (lane + 64 * u < (int)n) list[s0 + rk[u]] = (uint32_t)e[u];
     }
 }
 
-// Waves loop over the rows in list (at most kRowWave entries each): each wave sorts one row at a
-// time in its own kRowWave-entry slice of LDS, by rank (rows of at most kRankWave entries) or by
-// the bitonic network.  Within one wave every step only needs its LDS operations complete (a
-// wavefront fence), never a workgroup barrier.
-__global__ __launch_bounds__(kRowSortThreads) void k_row_sort_wave(const uint32_t *__restrict__ row_start,
-                                                                   const uint32_t *__restrict__ row_count,
-                                                                   uint32_t *__restrict__ skeys,
-                                                                   uint32_t *__restrict__ svals,
-                                                                   const uint32_t *__restrict__ list,
-                                                                   const uint32_t *__restrict__ count)
-{
-    __shared__ __align__(16) unsigned long long lds[(kRowSortThreads / 64) * kRowWave];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    unsigned long long *sk = lds + wv * kRowWave;
-    const uint32_t nb = *count;
-    const uint32_t nwaves = gridDim.x * (kRowSortThreads / 64);
-    for (uint32_t b = blockIdx.x * (kRowSortThreads / 64) + wv; b < nb; b += nwaves) {
-        const uint32_t r = list[b];
-        const uint32_t n = row_count[r];
-        const uint32_t s0 = row_start[r];
-        if (n <= (uint32_t)kRankWave) {
-            // rows of at most kRankWave entries (more than kRowSmall): by rank
-            switch ((n + 63) >> 6) {
-            case 1: rank_row<1>(skeys, svals, s0, n, sk, lane); break;
-            case 2: rank_row<2>(skeys, svals, s0, n, sk, lane); break;
-            case 3: rank_row<3>(skeys, svals, s0, n, sk, lane); break;
-            default: rank_row<kRankWave / 64>(skeys, svals, s0, n, sk, lane); break;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // before the next row reuses sk
-            continue;
-        }
-        int np2 = 1;
-        while ((uint32_t)np2 < n) np2 <<= 1;
-        for (int i = lane; i < np2; i += 64) sk[i] = (uint32_t)i < n ? row_entry(skeys, svals, s0 + i) : ~0ull;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        for (int k = 2; k <= np2; k <<= 1)
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int t = lane; t < (np2 >> 1); t += 64) {
-                    const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
-                    const int l = i + j;
-                    const unsigned long long a = sk[i], c = sk[l];
-                    const bool up = (i & k) == 0;
-                    if ((a > c) == up) {
-                        sk[i] = c;
-                        sk[l] = a;
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            }
-        for (int i = lane; (uint32_t)i < n; i += 64) {
-            const unsigned long long e = sk[i];
-            skeys[s0 + i] = (uint32_t)(e >> 32);
-            svals[s0 + i] = (uint32_t)e;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // before the next row reuses sk
-    }
-}
-
-// Workgroups loop over the rows in big_list (more than kRowWave entries): up to kLocalSortMax
-// entries by the bitonic network in LDS, more by rank (each entry counts the row's smaller composites; all composites differ)
-// through the scratch arrays tkeys/tvals.
-__global__ __launch_bounds__(kRowSortThreads) void k_row_sort_big(const uint32_t *__restrict__ row_start,
-                                                                  const uint32_t *__restrict__ row_count,
-                                                                  uint32_t *__restrict__ skeys,
-                                                                  uint32_t *__restrict__ svals,
-                                                                  const uint32_t *__restrict__ big_list,
-                                                                  const uint32_t *__restrict__ big_count,
-                                                                  uint32_t *__restrict__ tkeys,
-                                                                  uint32_t *__restrict__ tvals)
+// The rows of workgroup b are b, b + gridDim.x, ...: neighbouring rows, which tend to be of a
+// size, go to different workgroups.  A thread completes its row's start and sorts it if it is
+// small; the workgroup's waves then take its rows of up to kRowWave entries, each wave in its own
+// slice of the LDS, by rank or by the bitonic network (within one wave every step only needs its LDS
+// operations complete: a wavefront fence, never a barrier); then the whole workgroup its larger rows:
+// up to kLocalSortMax entries by the bitonic network in LDS, more by rank (each entry counts the row's
+// smaller composites; all composites differ).
+//
+// Bound by latency: each row a load, its sort and a store.  One launch instead of three (a global list
+// of rows for each kind) and the composites in one 64-bit array instead of two of 32: 16 fields of
+// 2400x1200 (19200 rows, 1.6 million points), scatter 25 + sorts 40 us, now 21 + 32; 65536 rows of 3 points
+// 7.1 + 14.3 us, now 6.2 + 9.0.  Of 512 threads with slices of 1024 composites it took 41 and 8.9.
+__global__ __launch_bounds__(kRowThreads) void k_row_sort(int64_t nrows, const uint32_t *__restrict__ row_count,
+                                                          uint32_t *__restrict__ row_start,
+                                                          const uint32_t *__restrict__ tiles,
+                                                          const unsigned long long *__restrict__ comp,
+                                                          uint32_t *__restrict__ list)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned long long *sk = reinterpret_cast<unsigned long long *>(smem);
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t nb = *big_count;
-    for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x) {
-        const uint32_t r = big_list[b];
-        const uint32_t n = row_count[r];
-        const uint32_t s0 = row_start[r];
-        if (n <= (uint32_t)kLocalSortMax) {
-            int np2 = 1;
-            while ((uint32_t)np2 < n) np2 <<= 1;
-            for (int i = tid; i < np2; i += nt) sk[i] = (uint32_t)i < n ? row_entry(skeys, svals, s0 + i) : ~0ull;
-            __syncthreads();
-            block_bitonic(sk, np2);
-            for (int i = tid; (uint32_t)i < n; i += nt) {
-                const unsigned long long e = sk[i];
-                skeys[s0 + i] = (uint32_t)(e >> 32);
-                svals[s0 + i] = (uint32_t)e;
+    __shared__ uint32_t s_n[kRowThreads], s_at[kRowThreads];   // rows for a wave from the front, larger ones from the end
+    __shared__ uint32_t s_count[2];
+    unsigned long long *const skb = reinterpret_cast<unsigned long long *>(smem);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    unsigned long long *const sk = skb + wv * kRowWave;
+    for (int64_t q0 = 0; q0 * gridDim.x < nrows; q0 += kRowThreads) {
+        const int64_t r = blockIdx.x + (q0 + tid) * gridDim.x;
+        if (tid < 2) s_count[tid] = 0u;
+        __syncthreads();
+        uint32_t n = 0, s0 = 0;
+        if (r < nrows) {
+            n = row_count[r];
+            s0 = row_start[r] + tiles[r / kTile];
+            row_start[r] = s0;
+        }
+        if (n > (uint32_t)kRowSmall) {
+            const bool big = n > (uint32_t)kRowWave;
+            const uint32_t k = atomicAdd(&s_count[big], 1u), at = big ? kRowThreads - 1 - k : k;
+            s_n[at] = n;
+            s_at[at] = s0;
+            n = 0;
+        }
+        if (__any(n > 8)) small_row<16>(comp, list, s0, n);
+        else if (__any(n > 4)) small_row<8>(comp, list, s0, n);
+        else if (__any(n > 2)) small_row<4>(comp, list, s0, n);
+        else if (__any(n > 0)) small_row<2>(comp, list, s0, n);
+        __syncthreads();
+        const int nwave = s_count[0], nbig = s_count[1];
+        for (int b = wv; b < nwave; b += kRowThreads / 64) {
+            const uint32_t m = s_n[b], a = s_at[b];
+            if (m <= (uint32_t)kRankWave) {
+                switch ((m + 63) >> 6) {
+                case 1: rank_row<1>(comp, list, a, m, sk, lane); break;
+                case 2: rank_row<2>(comp, list, a, m, sk, lane); break;
+                case 3: rank_row<3>(comp, list, a, m, sk, lane); break;
+                default: rank_row<kRankWave / 64>(comp, list, a, m, sk, lane); break;
+                }
+            } else {
+                int np2 = 1;
+                while ((uint32_t)np2 < m) np2 <<= 1;
+                for (int i = lane; i < np2; i += 64) sk[i] = (uint32_t)i < m ? comp[a + i] : ~0ull;
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                for (int k = 2; k <= np2; k <<= 1)
+                    for (int j = k >> 1; j > 0; j >>= 1) {
+                        for (int t = lane; t < (np2 >> 1); t += 64) {
+                            const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
+                            const int l = i + j;
+                            const unsigned long long x = sk[i], y = sk[l];
+                            const bool up = (i & k) == 0;
+                            if ((x > y) == up) {
+                                sk[i] = y;
+                                sk[l] = x;
+                            }
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    }
+                for (int i = lane; (uint32_t)i < m; i += 64) list[a + i] = (uint32_t)sk[i];
             }
-        } else {
-            for (uint32_t i = tid; i < n; i += nt) {
-                const unsigned long long ei = row_entry(skeys, svals, s0 + i);
-                uint32_t rank = 0;
-                for (uint32_t j = 0; j < n; ++j) rank += row_entry(skeys, svals, s0 + j) < ei;
-                tkeys[s0 + rank] = (uint32_t)(ei >> 32);
-                tvals[s0 + rank] = (uint32_t)ei;
-            }
-            __syncthreads();
-            for (uint32_t i = tid; i < n; i += nt) {
-                skeys[s0 + i] = tkeys[s0 + i];
-                svals[s0 + i] = tvals[s0 + i];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // before the next row reuses sk
+        }
+        for (int b = 0; b < nbig; ++b) {
+            const uint32_t m = s_n[kRowThreads - 1 - b], a = s_at[kRowThreads - 1 - b];
+            __syncthreads();   // the LDS is free
+            if (m <= (uint32_t)kLocalSortMax) {
+                int np2 = 1;
+                while ((uint32_t)np2 < m) np2 <<= 1;
+                for (int i = tid; i < np2; i += kRowThreads) skb[i] = (uint32_t)i < m ? comp[a + i] : ~0ull;
+                __syncthreads();
+                block_bitonic(skb, np2);
+                for (int i = tid; (uint32_t)i < m; i += kRowThreads) list[a + i] = (uint32_t)skb[i];
+            } else {
+                for (uint32_t i = tid; i < m; i += kRowThreads) {
+                    const unsigned long long e = comp[a + i];
+                    uint32_t rank = 0;
+                    for (uint32_t j = 0; j < m; ++j) rank += comp[a + j] < e;
+                    list[a + rank] = (uint32_t)e;
+                }
             }
         }
-        __syncthreads();   // the next row reuses sk / reads what this one wrote
+        __syncthreads();   // the lists and the LDS are reused
     }
 }
 
 }  // namespace
 
-int64_t scan_temp_elems(int64_t n)
-{
-    int64_t total = 0;
-    while (n > kTile) {
-        n = cdiv(n, kTile);
-        total += n;
-    }
-    return total + 1;
-}
+int64_t scan_tiles(int64_t n) { return n > 0 ? cdiv(n, kTile) : 1; }
 
-int scan_exclusive(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *tmp, hipStream_t stream)
+int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, const uint32_t *d_keys,
+                    const uint32_t *d_slot, int64_t npoints, uint32_t *d_row_start, const uint32_t *d_row_count,
+                    int64_t nrows, uint32_t *d_tiles, uint32_t *d_done, unsigned long long *d_comp, uint32_t *d_list,
+                    hipStream_t stream)
 {
-    if (n <= 0) return FB_OK;
-    const int64_t ntiles = cdiv(n, kTile);
-    if (ntiles == 1) {
-        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kThreads), 0, stream, in, out, (uint32_t *)nullptr, n);
+    if (nrows <= 0) return FB_OK;
+    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)scan_tiles(nrows)), dim3(kThreads), 0, stream, d_row_count,
+                       d_row_start, nrows, d_tiles, d_done);
+    FB_HIP_CHECK(hipGetLastError());
+    if (npoints > 0) {
+        hipLaunchKernelGGL(k_row_scatter, dim3((unsigned)cdiv(npoints, kThreads)), dim3(kThreads), 0, stream, d_fields,
+                           d_pt_prefix, nfields, npoints, d_keys, d_slot, (const uint32_t *)d_row_start,
+                           (const uint32_t *)d_tiles, d_comp);
         FB_HIP_CHECK(hipGetLastError());
-        return FB_OK;
     }
-    uint32_t *sums = tmp;
-    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)ntiles), dim3(kThreads), 0, stream, in, out, sums, n);
-    FB_HIP_CHECK(hipGetLastError());
-    int rc = scan_exclusive(sums, sums, ntiles, tmp + ntiles, stream);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)cdiv(n, kThreads)), dim3(kThreads), 0, stream, out,
-                       (const uint32_t *)sums, n);
-    FB_HIP_CHECK(hipGetLastError());
-    return FB_OK;
-}
-
-int local_sort_max() { return kLocalSortMax; }
-
-int row_bucket_sort(const uint32_t *d_keys, const uint32_t *d_slot, const uint32_t *d_rowg, int64_t npoints,
-                    const uint32_t *d_row_start, const uint32_t *d_row_count, int64_t nrows, uint32_t *d_skeys,
-                    uint32_t *d_svals, uint32_t *d_big_list, uint32_t *d_big_count, uint32_t *d_tkeys,
-                    uint32_t *d_tvals, hipStream_t stream)
-{
-    if (npoints <= 0 || nrows <= 0) return FB_OK;
-    hipLaunchKernelGGL(k_row_scatter, dim3((unsigned)cdiv(npoints, kThreads)), dim3(kThreads), 0, stream, npoints,
-                       d_keys, d_slot, d_rowg, d_row_start, d_skeys, d_svals);
-    FB_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_row_sort_small, dim3((unsigned)cdiv(nrows, kThreads)), dim3(kThreads), 0, stream, nrows,
-                       d_row_start, d_row_count, d_skeys, d_svals, d_big_list, d_big_count);
-    FB_HIP_CHECK(hipGetLastError());
-    const int64_t wgrid = std::min<int64_t>(cdiv(nrows, kRowSortThreads / 64), 2048);
-    hipLaunchKernelGGL(k_row_sort_wave, dim3((unsigned)wgrid), dim3(kRowSortThreads), 0, stream, d_row_start,
-                       d_row_count, d_skeys, d_svals, (const uint32_t *)d_big_list, (const uint32_t *)d_big_count);
-    FB_HIP_CHECK(hipGetLastError());
-    const int64_t grid = std::min<int64_t>(nrows, 1024);
-    hipLaunchKernelGGL(k_row_sort_big, dim3((unsigned)grid), dim3(kRowSortThreads),
-                       (size_t)kLocalSortMax * sizeof(unsigned long long), stream, d_row_start, d_row_count, d_skeys,
-                       d_svals, (const uint32_t *)(d_big_list + nrows), (const uint32_t *)(d_big_count + 1), d_tkeys,
-                       d_tvals);
+    hipLaunchKernelGGL(k_row_sort, dim3((unsigned)std::min<int64_t>(nrows, kRowGrid)), dim3(kRowThreads),
+                       (size_t)kLocalSortMax * sizeof(unsigned long long), stream, nrows, d_row_count, d_row_start,
+                       (const uint32_t *)d_tiles, (const unsigned long long *)d_comp, d_list);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
@@ -505,11 +568,13 @@ int field_sort_init()
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {
-        err = hipFuncSetAttribute((const void *)k_field_sort, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  kLocalSortMax * (int)sizeof(unsigned long long));
-        if (err == hipSuccess)
-            err = hipFuncSetAttribute((const void *)k_row_sort_big, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      kLocalSortMax * (int)sizeof(unsigned long long));
+        const int lds = (kLocalSortMax + kRankStep) * (int)sizeof(unsigned long long);
+        const void *fns[] = {(const void *)k_field_sort<1, false>, (const void *)k_field_sort<2, false>,
+                             (const void *)k_field_sort<3, false>, (const void *)k_field_sort<1, true>,
+                             (const void *)k_field_sort<2, true>,  (const void *)k_field_sort<3, true>,
+                             (const void *)k_row_sort};
+        for (const void *fn : fns)
+            if (err == hipSuccess) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     });
     if (err != hipSuccess) {
         (void)hipGetLastError();
@@ -519,19 +584,36 @@ int field_sort_init()
     return FB_OK;
 }
 
-int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int max_n,
-                      const uint32_t *d_keys, const uint32_t *d_row_count, uint32_t *d_row_start,
-                      uint32_t *d_out_vals, hipStream_t stream)
+int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int dim, int max_n,
+                      int max_rows, const double *d_pts, const double *d_val, bool raw, double *d_offsets,
+                      uint32_t *d_row_count, uint32_t *d_row_start, uint32_t *d_out_vals, PointRec *d_rec,
+                      InjectRec *d_irec, const ZeroRange (&zero)[2], hipStream_t stream)
 {
     if (nfields <= 0) return FB_OK;
-    if (max_n > kLocalSortMax) {
-        set_error("field sort: a field has more than " + std::to_string(kLocalSortMax) + " points");
+    if (max_n > kLocalSortMax || max_rows > kLocalRowsMax) {
+        set_error("field sort: a field has more than " + std::to_string(kLocalSortMax) + " points or " +
+                  std::to_string(kLocalRowsMax) + " x-lines");
         return FB_ERR_UNSUPPORTED;
     }
     int np2 = 1;
     while (np2 < max_n) np2 <<= 1;
-    hipLaunchKernelGGL(k_field_sort, dim3(nfields), dim3(kLocalSortThreads), (size_t)np2 * 8, stream, d_fields,
-                       d_pt_prefix, d_keys, d_row_count, d_row_start, d_out_vals);
+    FieldSortArgs A{d_fields,   d_pt_prefix, d_pts, d_val,  d_offsets,          d_row_count, d_row_start,
+                    d_out_vals, d_rec,       d_irec, {zero[0], zero[1]}, nfields, np2, raw ? 1 : 0};
+    int64_t grid = nfields;
+    for (const ZeroRange &z : zero) grid += zero_blocks<kLocalSortThreads, kSortZeroPer>(z);
+    const size_t lds = (size_t)(np2 + kRankStep) * 8;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kLocalSortThreads), lds, stream, A);
+    };
+    if (d_irec) {
+        if (dim == 1) launch(k_field_sort<1, true>);
+        else if (dim == 2) launch(k_field_sort<2, true>);
+        else launch(k_field_sort<3, true>);
+    } else {
+        if (dim == 1) launch(k_field_sort<1, false>);
+        else if (dim == 2) launch(k_field_sort<2, false>);
+        else launch(k_field_sort<3, false>);
+    }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
