@@ -1525,7 +1525,7 @@ int fb_plan_backward(fb_plan *P, const double *d_pts, const double *d_val, const
         rc = run_pass(P, a, false, nullptr, nullptr, a == 0 ? const_cast<float *>(d_out) : nullptr,
                       a == 0 ? const_cast<float *>(d_wsave) : nullptr, 0, s, a == 0 ? d_gout : nullptr);
     if (!rc)
-        rc = launch_adj_gather(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, d_pts, d_val, P->d_offsets,
+        rc = launch_adj_gather(P->d_fields, P->d_pt_prefix, P->nfields, P->dim, P->npoints, d_pts, d_val, P->d_offsets,
                                P->d_v, P->d_w, P->dim >= 2 ? P->d_pass[1] : nullptr, d_gval, d_gpts, s);
     const int rc2 = P->mark_use(s);
     return rc ? rc : rc2;

@@ -1665,12 +1665,14 @@ __global__ __launch_bounds__(kBlock) void k_f32_to_f64(const float *__restrict__
 // normalisation (1/(K+2 alpha))^n per axis in both V and W; applying the same scaled
 // operator to a = g/W_scaled gives the same A, so the gradient needs no rescaling.
 
-// a and b at every node of the batch in the cell layout; zero where the forward result
-// is NaN (masked) or the incoming gradient is NaN, and in the alignment gaps.
-// Transposed injection: one thread per point gathers A and Bb at its 2^dim corners.
+// Transposed injection: one thread per point gathers A and Bb at its 2^DIM corners.
 // Points dropped by the injection (outside the grid, NaN) get zero gradients.  (Taking the
 // points in the forward's sorted order makes the A, Bb reads local but the point reads and
 // gradient writes scattered; measured slower.)
+//
+// Bound by the random reads' latency: all corners of a point are loaded before the first is used.
+// 1.6 million points on 16 fields of 2400x1200: corner by corner 99 us, now 67.
+template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_adj_gather(const FieldDev *__restrict__ fields,
                                                        const int64_t *__restrict__ pt_prefix, int nfields,
                                                        int64_t npoints, const double *__restrict__ pts,
@@ -1680,40 +1682,51 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(const FieldDev *__restric
                                                        const PassField *__restrict__ pass_y,
                                                        double *__restrict__ gval, double *__restrict__ gpts)
 {
+    constexpr int NC = 1 << DIM;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= npoints) return;
+    double c[DIM];
+#pragma unroll
+    for (int m = 0; m < DIM; ++m) c[m] = pts[i * DIM + m];
+    const double v = val[i];
     const int f = find_seg(pt_prefix, nfields, i);
     const FieldDev &F = fields[f];
-    const int dim = F.dim;
     // A and B of a 2D field whose y pass ran on the blocked intermediate are (A, B) pairs
     // (adj_pair_index), the pairs of rows y % 8 < 4 in A's field and the others in Bb's
-    const bool blocked = pass_y && pass_y[f].blocked == kBlockedIn;
+    const bool blocked = DIM == 2 && pass_y[f].blocked == kBlockedIn;
     PointPos pp;
-    const bool inside = point_pos(F, pts + i * dim, pp);
     double gv = 0.0, gp[3] = {0.0, 0.0, 0.0};
-    if (inside) {
-        const double vk = val[i] - offsets[f];
+    if (point_pos(F, c, pp)) {
+        const double vk = v - offsets[f];
         const int64_t W = F.size[0], H = F.size[1];
-        const int corners = 1 << dim;
-        for (int cb = 0; cb < corners; ++cb) {
-            const int bx = cb & 1, by = (cb >> 1) & 1, bz = (cb >> 2) & 1;
-            double a, b;
-            if (blocked) {
-                const int64_t y = pp.i[1] + by;
+        float ca[NC], cb[NC];
+        if (blocked) {
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                const int64_t y = pp.i[1] + ((q >> 1) & 1);
                 const float2 ab = *reinterpret_cast<const float2 *>((y & 4 ? Bb : A) + F.cell_off +
-                                                                    adj_pair_index(y, pp.i[0] + bx, W));
-                a = (double)ab.x;
-                b = (double)ab.y;
-            } else {
-                const int64_t cell = F.cell_off + ((pp.i[2] + bz) * H + (pp.i[1] + by)) * W + (pp.i[0] + bx);
-                a = (double)A[cell];
-                b = (double)Bb[cell];
+                                                                    adj_pair_index(y, pp.i[0] + (q & 1), W));
+                ca[q] = ab.x;
+                cb[q] = ab.y;
             }
+        } else {
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                const int64_t cell = F.cell_off + ((pp.i[2] + (q >> 2)) * H + (pp.i[1] + ((q >> 1) & 1))) * W +
+                                     (pp.i[0] + (q & 1));
+                ca[q] = A[cell];
+                cb[q] = Bb[cell];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const int bx = q & 1, by = (q >> 1) & 1, bz = q >> 2;
+            const double a = (double)ca[q], b = (double)cb[q];
             const double fx = bx ? pp.w[0] : 1.0 - pp.w[0];
-            const double fy = dim >= 2 ? (by ? pp.w[1] : 1.0 - pp.w[1]) : 1.0;
-            const double fz = dim >= 3 ? (bz ? pp.w[2] : 1.0 - pp.w[2]) : 1.0;
+            const double fy = DIM >= 2 ? (by ? pp.w[1] : 1.0 - pp.w[1]) : 1.0;
+            const double fz = DIM >= 3 ? (bz ? pp.w[2] : 1.0 - pp.w[2]) : 1.0;
             const double sx = bx ? 1.0 : -1.0, sy = by ? 1.0 : -1.0, sz = bz ? 1.0 : -1.0;
-            gv += corner_weight(dim, pp, bx, by, bz) * a;
+            gv += corner_weight(DIM, pp, bx, by, bz) * a;
             const double t = vk * a + b;
             gp[0] += sx * fy * fz * t;
             gp[1] += fx * sy * fz * t;
@@ -1721,8 +1734,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(const FieldDev *__restric
         }
     }
     gval[i] = gv;
-    if (gpts)
-        for (int m = 0; m < dim; ++m) gpts[i * dim + m] = gp[m] / F.step[m];
+    if (gpts) {
+#pragma unroll
+        for (int m = 0; m < DIM; ++m) gpts[i * DIM + m] = gp[m] / F.step[m];
+    }
 }
 
 inline unsigned nblocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -1969,13 +1984,18 @@ int launch_fast_pass(int kind, bool inject, int seg, const FieldDev *d_fields, c
     return FB_OK;
 }
 
-int launch_adj_gather(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
+int launch_adj_gather(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int dim, int64_t npoints,
                       const double *d_pts, const double *d_val, const double *d_offsets, const float *d_A,
                       const float *d_Bb, const PassField *d_pass_y, double *d_gval, double *d_gpts, hipStream_t s)
 {
     if (npoints <= 0) return FB_OK;
-    hipLaunchKernelGGL(k_adj_gather, dim3(nblocks(npoints)), dim3(kBlock), 0, s, d_fields, d_pt_prefix, nfields,
-                       npoints, d_pts, d_val, d_offsets, d_A, d_Bb, d_pass_y, d_gval, d_gpts);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nblocks(npoints)), dim3(kBlock), 0, s, d_fields, d_pt_prefix, nfields, npoints,
+                           d_pts, d_val, d_offsets, d_A, d_Bb, d_pass_y, d_gval, d_gpts);
+    };
+    if (dim == 1) launch(k_adj_gather<1>);
+    else if (dim == 2) launch(k_adj_gather<2>);
+    else launch(k_adj_gather<3>);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }

@@ -91,7 +91,7 @@ int launch_fast_pass(int kind, bool inject, int seg, const FieldDev *d_fields, c
                      float *d_wsave, int final_pass, const float *d_adj_g, hipStream_t stream);
 
 // fb_kernels.hip -- adjoint of the FP32C batch
-int launch_adj_gather(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
+int launch_adj_gather(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int dim, int64_t npoints,
                       const double *d_pts, const double *d_val, const double *d_offsets, const float *d_A,
                       const float *d_Bb, const PassField *d_pass_y, double *d_gval, double *d_gpts,
                       hipStream_t stream);
