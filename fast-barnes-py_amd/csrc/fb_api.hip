@@ -1004,7 +1004,8 @@ int build_pass(fb_plan *P, int axis, std::vector<PassWork> &work, std::vector<Pa
             const int64_t nlines = H * D;
             for (int64_t l0 = 0; l0 < nlines; l0 += lines)
                 for (int c = 0; c < nch; ++c)
-                    items.push_back({f, (int32_t)std::min<int64_t>(lines, nlines - l0), l0 * W, c});
+                    items.push_back({f, (int32_t)std::min<int64_t>(lines, nlines - l0), l0 * W, c,
+                                     P->dim >= 3 ? (int32_t)H : 0, (uint32_t)l0, (uint32_t)(F.xline_off + l0)});
         } else if (axis == 1) {
             p.line_stride = 1;
             p.elem_stride = W;
@@ -1239,7 +1240,7 @@ int plan_sort(fb_plan *P, const double *pts, const double *val, bool raw, hipStr
     // whole 16-byte words: the row counts' allocation is a multiple of 256 bytes
     const ZeroRange counts{(uint4 *)P->d_line_count, (P->nxlines + 3) / 4};
     if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->max_n, val, P->d_off_part, P->d_done, {counts, vg, wg}, s)) ||
-        (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->max_n, P->npoints, pts, P->d_keys,
+        (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->max_n, P->npoints, pts, val, P->d_keys,
                                 P->d_line_count, P->d_slot, P->max_rows, P->d_rec, P->d_off_part, P->d_offsets, s)) ||
         (rc = row_bucket_sort(P->d_fields, P->d_pt_prefix, P->nfields, P->d_keys, P->d_slot, P->npoints,
                               P->d_line_start, P->d_line_count, P->nxlines, P->d_tiles, P->d_done, P->d_comp, P->d_list,

@@ -65,7 +65,11 @@ struct PassWork {
     int32_t nlines;
     int64_t base;
     int32_t chunk = 0;
-    int32_t pad_ = 0;
+    // injecting passes: the rows of a plane (3D, else 0), the first line's index in the field and
+    // its row (x-line of the plan), so that the row starts are read without the field's descriptor
+    int32_t plane = 0;
+    uint32_t line = 0;
+    uint32_t row = 0;
 };
 
 // Doubles per line in the LDS of the prefix pass: positions -T-1 .. lpl*seg+T+1, rounded up
@@ -139,7 +143,7 @@ __host__ __device__ inline int64_t adj_pair_index(int64_t y, int64_t x, int64_t 
 // A point's grid position as the FP32C injection uses it, formed once per point by the
 // point-key kernels (point_pos): its base cell along x and its fractional offsets per axis.
 struct PointRec {
-    double w[3];
+    double w[3];   // 1D, 2D: w[2] is the point's value, so that one read gives both
     int32_t xi;
     int32_t pad_;
 };

@@ -151,6 +151,7 @@ __device__ __forceinline__ double corner_weight(int dim, const PointPos &pp, int
 __global__ __launch_bounds__(kBlock) void k_point_keys(const FieldDev *__restrict__ fields,
                                                        const int64_t *__restrict__ pt_prefix, int nfields,
                                                        int64_t npoints, const double *__restrict__ pts,
+                                                       const double *__restrict__ val,
                                                        uint32_t *__restrict__ keys, uint32_t *__restrict__ row_count,
                                                        uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
                                                        int64_t nkb, const double *__restrict__ part, int nchunk,
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(kBlock) void k_point_keys(const FieldDev *__restric
     }
     const int64_t row = pp.i[2] * F.size[1] + pp.i[1];
     keys[i] = (uint32_t)(F.cell_off + row * F.size[0] + pp.i[0]);
-    if (rec) rec[i] = PointRec{{pp.w[0], pp.w[1], pp.w[2]}, (int32_t)pp.i[0], 0};
+    if (rec) rec[i] = PointRec{{pp.w[0], pp.w[1], F.dim >= 3 ? pp.w[2] : val[i]}, (int32_t)pp.i[0], 0};
     slot[i] = atomicAdd(&row_count[F.xline_off + row], 1u);
 }
 
@@ -189,6 +190,7 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
                                                             const int64_t *__restrict__ pt_prefix, int nfields,
                                                             int64_t npoints, int ppt, int nbins,
                                                             const double *__restrict__ pts,
+                                                            const double *__restrict__ val,
                                                             uint32_t *__restrict__ keys,
                                                             uint32_t *__restrict__ row_count,
                                                             uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
             }
             const int64_t row = ci[2] * gsz[1] + ci[1];
             keys[i] = (uint32_t)(gcell + row * gsz[0] + ci[0]);
-            if (rec) rec[i] = PointRec{{w[0], w[1], w[2]}, (int32_t)ci[0], 0};
+            if (rec) rec[i] = PointRec{{w[0], w[1], dim >= 3 ? w[2] : val[i]}, (int32_t)ci[0], 0};
             const int64_t grow = gxl + row;
             if (span >= 0) {
                 rr[k] = (int)(grow - rbase);
@@ -307,38 +309,6 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
         if (rr[k] < 0) continue;
         const int64_t i = p0 + (int64_t)k * kBlock + threadIdx.x;
         slot[i] = hist[rr[k]] + lr[k];
-    }
-}
-
-// The sub-streams of x-line (y, z): for q < 2*nrows, the points of base row (y - dy, z - dz)
-// contribute their corner (bx, dy, dz) at x = base x + bx, with bx = q & 1, dy = (q >> 1) & 1,
-// dz = q >> 2.  Within a base row the sorted points ascend in base x (point order for equal
-// x), so every sub-stream ascends in target cell.
-__device__ __forceinline__ int source_rows(int dim) { return dim >= 3 ? 4 : (dim == 2 ? 2 : 1); }
-
-__device__ __forceinline__ void line_streams(const FieldDev &F, int64_t line, bool enable,
-                                             const uint32_t *__restrict__ row_start,
-                                             const uint32_t *__restrict__ row_count, uint32_t (&rs)[8],
-                                             uint32_t (&rc)[8])
-{
-    // sub-stream q reads base row (y - dy, z - dz) with dy = (q >> 1) & 1, dz = q >> 2 for its
-    // corner column bx = q & 1: both corner columns of a row share the row's range, loaded
-    // once; (y, z) are formed once per line (a 2D line index is y itself)
-    const int nsub = 2 * source_rows(F.dim);
-    const int64_t H = F.size[1];
-    const int64_t y = F.dim >= 3 ? line % H : line;
-    const int64_t z = F.dim >= 3 ? line / H : 0;
-#pragma unroll
-    for (int q = 0; q < 8; q += 2) {
-        const int dy = (q >> 1) & 1, dz = q >> 2;
-        uint32_t st = 0, ct = 0;
-        if (enable && q < nsub && y - dy >= 0 && z - dz >= 0) {
-            const int64_t row = line - dy - dz * H;
-            st = row_start[F.xline_off + row];
-            ct = row_count[F.xline_off + row];
-        }
-        rs[q] = rs[q + 1] = st;
-        rc[q] = rc[q + 1] = ct;
     }
 }
 
@@ -1031,79 +1001,113 @@ __device__ __forceinline__ double dpp_from_next(double v)
     return __hiloint2double(dpp_from_next(__double2hiint(v)), dpp_from_next(__double2loint(v)));
 }
 
-// Deterministic fused injection of one line's points into its float32 row (element x at
-// row[x]).  The line's sub-streams (line_streams: one base row, one corner column),
+// Deterministic fused injection of one line's points into its float32 row.  For s < 4 (2 without
+// planes), the points of base row (y - dy, z - dz), dy = s & 1, dz = s >> 1, contribute their corners
+// (0, dy, dz) and (1, dy, dz) at x = base x and base x + 1: two sub-streams, in which the points
+// ascend in base x (point order for equal x) and so in target cell.  The line's sub-streams,
 // concatenated, are taken in chunks of up to 64 entries by the line's first `iw` lanes
 // (`injector`).  A run sum over adjacent lanes of equal target cell (in lane order) gives
 // each run's total to its first lane.  Equal cells adjacent in one
 // sub-stream form one run; a cell can head two runs of a chunk only from different
 // sub-streams, so the heads add their totals in one round per sub-stream of the head
 // (program order), without conflicts.  The result does not depend on timing.  Called by
-// every thread of the workgroup (wave-wide shuffles).
-__device__ __forceinline__ void inject_line(const FieldDev &F, int64_t line_in_field, bool injector, int iw, int sid,
-                                            int fsel, double off, const uint32_t *__restrict__ vals,
-                                            const uint32_t *__restrict__ line_start,
-                                            const uint32_t *__restrict__ line_count, const PointRec *__restrict__ rec,
-                                            const double *__restrict__ val, float *row, int lo, int len)
-{
+// every thread of the workgroup (wave-wide ballots).
+//
+// Bound by its instructions, some hundred per chunk and wave, which every line pays at least once: the
+// x pass without it 548 us of 650 (64 fields of 2400x1200, 6 points to a row), 534 of 733 (96 uneven
+// fields).  Row ranges without a division, entries found row by row, chunks counted by ballots, runs
+// summed up to their ends and the value beside the position (1D, 2D): x 650 -> 625, 733 -> 670 us, and
+// 162 -> 157 for 512x512x128 with 200000 points.
+struct LineInjection {
+    uint32_t start[4], count[4];   // the base rows' ranges of the sorted list
+    uint32_t total;                // entries of the line
+
+    // the row ranges, before the line is cleared
+    __device__ __forceinline__ void begin(const PassWork &wk, int my_line, bool injector,
+                                          const uint32_t *__restrict__ line_start,
+                                          const uint32_t *__restrict__ line_count)
+    {
+        const uint32_t line = wk.line + my_line, row = wk.row + my_line, H = wk.plane;
+        const uint32_t y = H ? line % H : line, z = H ? line / H : 0u;   // a 2D line is y itself
+        total = 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const uint32_t dy = s & 1, dz = s >> 1;
+            start[s] = count[s] = 0;
+            if (s < 2 || H) {
+                if (injector && y >= dy && z >= dz) {
+                    const uint32_t r = row - dy - dz * H;
+                    start[s] = line_start[r];
+                    count[s] = line_count[r];
+                }
+                total += 2 * count[s];
+            }
+        }
+    }
+
     // row[x - lo] receives cell x of the line for x in [lo, lo + len) (a chunk of a long line);
     // cells outside are skipped
-    const int nsub = 2 * source_rows(F.dim);
-    uint32_t rsq[8], rcq[8], pre[9];
-    line_streams(F, line_in_field, injector, line_start, line_count, rsq, rcq);
-    pre[0] = 0;
+    __device__ __forceinline__ void add(int dim, bool planes, int iw, int sid, int fsel, double off,
+                                        const uint32_t *__restrict__ vals, const PointRec *__restrict__ rec,
+                                        const double *__restrict__ val, float *row, int lo, int len)
+    {
+        // This lane's entry e: its sub-stream (2 * row + corner column) and its slot in the sorted
+        // point list.
+        auto entry = [&](uint32_t e, int &hq, uint32_t &src) {
+            uint32_t st = start[0], ct = count[0];
+            hq = 0;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) pre[q + 1] = pre[q] + rcq[q];
-    int nch = (int)((pre[8] + iw - 1) / iw);
-    for (int d = 32; d >= 1; d >>= 1) nch = max(nch, __shfl_xor(nch, d));
-    // This lane's entry of chunk ch: its sub-stream and its slot in the sorted point list.
-    auto entry = [&](int ch, int &hq, uint32_t &src) {
-        const uint32_t e = (uint32_t)ch * iw + sid;
-        hq = 0;
-        src = 0;
-        if (!injector || e >= pre[8]) return false;
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            if (e >= pre[q] && e < pre[q + 1]) {
-                hq = q;
-                src = rsq[q] + (e - pre[q]);
+            for (int s = 1; s < 4; ++s)
+                if (s < 2 || planes) {
+                    const bool on = hq == 2 * (s - 1) && e >= 2 * ct;   // past row s - 1
+                    e -= on ? 2 * ct : 0u;
+                    st = on ? start[s] : st;
+                    ct = on ? count[s] : ct;
+                    hq = on ? 2 * s : hq;
+                }
+            const bool bx = e >= ct;
+            src = st + e - (bx ? ct : 0u);
+            hq += bx;
+        };
+        // Software pipeline over the chunks: while chunk ch is summed, the point data of chunk ch+1
+        // and the point index of chunk ch+2 are in flight.
+        auto fetch_index = [&](uint32_t e, bool &ok, int &hq, uint32_t &p) {
+            ok = e < total;
+            hq = 0;
+            p = 0;
+            if (ok) {
+                uint32_t src;
+                entry(e, hq, src);
+                p = vals[src];
             }
-        return true;
-    };
-    struct PointData {
-        PointRec r;
-        double v;
-    };
-    auto load_point = [&](bool ok, uint32_t p, PointData &o) {
-        o.r = PointRec{{0.0, 0.0, 0.0}, 0, 0};
-        o.v = 0.0;
-        if (!ok) return;
-        o.r = rec[p];
-        o.v = val[p];
-    };
-    // Software pipeline over the chunks: while chunk ch is summed, the point data of chunk ch+1
-    // and the point index of chunk ch+2 are in flight.
-    auto fetch_index = [&](int ch, bool &ok, int &hq, uint32_t &p) {
-        uint32_t src;
-        ok = entry(ch, hq, src);
-        p = ok ? vals[src] : 0u;
-    };
-    bool ok_a, ok_b;
-    int hq_a, hq_b;
-    uint32_t p_a, p_b;
-    PointData pd_a;
-    fetch_index(0, ok_a, hq_a, p_a);
-    load_point(ok_a, p_a, pd_a);
-    fetch_index(1, ok_b, hq_b, p_b);
-    for (int ch = 0; ch < nch; ++ch) {
-        const bool valid = ok_a;
-        const int hq = hq_a;
-        const PointData pd = pd_a;
-        ok_a = ok_b;
-        hq_a = hq_b;
-        load_point(ok_b, p_b, pd_a);
-        fetch_index(ch + 2, ok_b, hq_b, p_b);
-        {
+        };
+        struct PointData {
+            PointRec r;
+            double v;
+        };
+        auto load_point = [&](bool ok, uint32_t p, PointData &o) {
+            o.r = PointRec{{0.0, 0.0, 0.0}, 0, 0};
+            o.v = 0.0;
+            if (!ok) return;
+            o.r = rec[p];
+            if (planes) o.v = val[p];
+        };
+        const int lane = threadIdx.x & 63;
+        bool ok_a, ok_b;
+        int hq_a, hq_b;
+        uint32_t p_a, p_b, e = sid;
+        PointData pd_a;
+        fetch_index(e, ok_a, hq_a, p_a);
+        load_point(ok_a, p_a, pd_a);
+        fetch_index(e += iw, ok_b, hq_b, p_b);
+        while (__any(ok_a)) {   // the chunks ascend: a lane without an entry has none in later ones
+            const bool valid = ok_a;
+            const int hq = hq_a;
+            const PointData pd = pd_a;
+            ok_a = ok_b;
+            hq_a = hq_b;
+            load_point(ok_b, p_b, pd_a);
+            fetch_index(e += iw, ok_b, hq_b, p_b);
             int x = -1;
             double c = 0.0;
             if (valid) {
@@ -1114,39 +1118,36 @@ __device__ __forceinline__ void inject_line(const FieldDev &F, int64_t line_in_f
                     pp.w[m] = pd.r.w[m];
                 }
                 x = pd.r.xi + (hq & 1);
-                const double w = corner_weight(F.dim, pp, hq & 1, (hq >> 1) & 1, hq >> 2);
-                c = fsel ? w : w * (pd.v - off);
+                const double w = corner_weight(dim, pp, hq & 1, (hq >> 1) & 1, hq >> 2);
+                c = fsel ? w : w * ((planes ? pd.v : pd.r.w[2]) - off);
             }
-            // runs: maximal groups of adjacent lanes with equal cell; run id = inclusive count
-            // of run starts (the concatenated stream is not sorted, so equal cells further
-            // apart belong to different runs)
+            // runs: maximal groups of adjacent lanes with equal cell (the concatenated stream is
+            // not sorted, so equal cells further apart belong to different runs), each up to the
+            // next run's first lane
             const int px = dpp_from_prev(x);
             const bool start = sid == 0 || px != x;
-            const int lane = threadIdx.x & 63;
-            const int rid = __popcll(__ballot(start) & ((2ull << lane) - 1ull));
             // The run sum only where some run of this wave's chunk has more than one entry:
             // otherwise every lane is its own run and keeps c.  Each run's first lane adds the
             // contributions of the run's next lanes one at a time (DPP wave shifts, no LDS
-            // round trips), in lane order; runs are short, so this stops after a few steps.
-            if (__ballot(valid && !start)) {
+            // round trips), in lane order, until the longest run ends.
+            if (__any(valid && !start)) {
+                const unsigned long long next = (__ballot(start) >> lane) >> 1;
+                const int left = valid ? (next ? __builtin_ctzll(next) + 1 : 64 - lane) : 0;   // this lane's run from here on
                 double o = c;
-                int orid = rid;
-                for (int t = 1; t < iw; ++t) {
+                for (int t = 1; __any(t < left); ++t) {
                     o = dpp_from_next(o);
-                    orid = dpp_from_next(orid);
-                    const bool take = sid + t < iw && orid == rid;
-                    if (take) c += o;
-                    if (!__ballot(take)) break;
+                    if (t < left) c += o;
                 }
             }
-            const bool head = valid && start;
-            const bool here = head && x >= lo && x < lo + len;
+            const bool here = valid && start && x >= lo && x < lo + len;
             float *cell = row + (here ? x - lo : 0);
-            for (int q = 0; q < nsub; ++q)
-                if (here && hq == q) *cell = (float)((double)*cell + c);
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (q < 4 || planes)
+                    if (here && hq == q) *cell = (float)((double)*cell + c);
         }
     }
-}
+};
 
 // Orders the LDS accesses of one phase of a line pass before the next: a workgroup
 // barrier when a line spans several waves; a line within one wave needs only program order
@@ -1214,9 +1215,10 @@ __global__ __launch_bounds__(kFastBlock, 1) void k_fast_pass(
     // injection: the first (up to 64) lanes of each line
     const int iw = lpl < 64 ? lpl : 64;
     const bool injector = INJECT && line_ok && sid < iw;
-    const int64_t line_in_field = INJECT ? wk.base / F.size[0] + my_line : 0;
+    LineInjection inj;
 
     if (INJECT) {
+        inj.begin(wk, my_line, injector, line_start, line_count);
         // each line's lanes zero the line's left padding, cells and gap (the left padding is
         // the previous line's gap end, which that line also zeroes and never writes again:
         // zeros over zeros); lines past nl and the reserve after the w lines feed only
@@ -1269,8 +1271,7 @@ __global__ __launch_bounds__(kFastBlock, 1) void k_fast_pass(
 
     if (INJECT) {
         // a line's injection writes cells 0..L-1 of that line only
-        inject_line(F, line_in_field, injector, iw, sid, fsel, off, vals, line_start, line_count, rec, val,
-                    mine + my_line * lstride + pad, lo, L);
+        inj.add(F.dim, wk.plane != 0, iw, sid, fsel, off, vals, rec, val, mine + my_line * lstride + pad, lo, L);
         line_sync(lpl);
     }
 
@@ -1522,14 +1523,14 @@ __global__ __launch_bounds__(kFastBlock, 1) void k_prefix_pass(
     const double off = offsets[wk.field];
 
     if (INJECT) {
+        const int iw = lpl < 64 ? lpl : 64;
+        LineInjection inj;
+        inj.begin(wk, my_line, line_ok && sid < iw, line_start, line_count);
         float4 *z = reinterpret_cast<float4 *>(smem);
         const int nz = (2 * lines_cap * fstride) >> 2;
         for (int i = tid; i < nz; i += nthr) z[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
-        const int iw = lpl < 64 ? lpl : 64;
-        const int64_t line_in_field = wk.base / F.size[0] + my_line;
-        inject_line(F, line_in_field, line_ok && sid < iw, iw, sid, fsel, off, vals, line_start, line_count, rec, val,
-                    myX, 0, L);
+        inj.add(F.dim, wk.plane != 0, iw, sid, fsel, off, vals, rec, val, myX, 0, L);
     } else {
         if (adj_g)
             adjoint_load(out + F.out_off + wk.base, wsave + F.out_off + wk.base, adj_g + F.out_off + wk.base, off,
@@ -1783,8 +1784,8 @@ int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, cons
 }
 
 int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
-                      int64_t npoints, const double *d_pts, uint32_t *d_keys, uint32_t *d_row_count, uint32_t *d_slot,
-                      int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t s)
+                      int64_t npoints, const double *d_pts, const double *d_val, uint32_t *d_keys,
+                      uint32_t *d_row_count, uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t s)
 {
     if (nfields <= 0) return FB_OK;
     const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
@@ -1801,12 +1802,13 @@ int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
         const int nbins = max_rows <= kKeysBins ? kKeysBins : kKeysBinsMax;
         const int64_t per = ppt * kBlock, nkb = (npoints + per - 1) / per;
         hipLaunchKernelGGL(k_point_keys_hist, dim3((unsigned)(nkb + nfin)), dim3(kBlock), (size_t)nbins * 4, s,
-                           d_fields, d_pt_prefix, nfields, npoints, (int)ppt, nbins, d_pts, d_keys, d_row_count, d_slot,
+                           d_fields, d_pt_prefix, nfields, npoints, (int)ppt, nbins, d_pts, d_val, d_keys, d_row_count, d_slot,
                            d_rec, nkb, d_part, nchunk, d_offsets);
     } else {
         const int64_t nkb = npoints > 0 ? nblocks(npoints) : 0;
         hipLaunchKernelGGL(k_point_keys, dim3((unsigned)(nkb + nfin)), dim3(kBlock), 0, s, d_fields, d_pt_prefix,
-                           nfields, npoints, d_pts, d_keys, d_row_count, d_slot, d_rec, nkb, d_part, nchunk, d_offsets);
+                           nfields, npoints, d_pts, d_val, d_keys, d_row_count, d_slot, d_rec, nkb, d_part, nchunk,
+                           d_offsets);
     }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;

@@ -40,8 +40,8 @@ int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, const d
 int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
                       uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t stream);
 int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
-                      int64_t npoints, const double *d_pts, uint32_t *d_keys, uint32_t *d_row_count, uint32_t *d_slot,
-                      int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t stream);
+                      int64_t npoints, const double *d_pts, const double *d_val, uint32_t *d_keys,
+                      uint32_t *d_row_count, uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t stream);
 
 // fb_kernels.hip -- FP64 path with the reference's operation order
 // Each sorted entry's FP64 injection record (row buckets).

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
 #pragma unroll
                         for (int m = 0; m < DIM; ++m) w[k][m] = pp.w[m];
                     } else {
-                        A.rec[p0 + i] = PointRec{{pp.w[0], pp.w[1], pp.w[2]}, xi[k], 0};
+                        A.rec[p0 + i] = PointRec{{pp.w[0], pp.w[1], DIM >= 3 ? pp.w[2] : v[k]}, xi[k], 0};
                     }
                 }
             }
