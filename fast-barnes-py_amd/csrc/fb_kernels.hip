@@ -740,6 +740,14 @@ __device__ __forceinline__ void stage_store(float *__restrict__ lin, int s, int 
     }
 }
 
+// Four floats that this pass reads once, from a line that no other workgroup reads: nontemporal.
+__device__ __forceinline__ float4 load_once(const float *p)
+{
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const f32x4 x = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p));
+    return make_float4(x.x, x.y, x.z, x.w);
+}
+
 __device__ __forceinline__ bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 // global tile <-> LDS.  Tile: nl lines of length L; element (l, j) at g[l*ls + j*es] maps
@@ -868,7 +876,11 @@ __device__ __forceinline__ void blocked_store_rows(float *__restrict__ g, int64_
 // y-pass load of the columns x0 .. x0+nl-1 (nl a multiple of 4) of both intermediate fields
 // from the blocked layout into LDS lines (line l, element j at lds[l*lstride + j]).  Thread t
 // takes column group t % (nl/4) and rows t / (nl/4) + k*rstep, k < kBlkRows (the host checks
-// that they cover the column); all loads are issued before the first LDS write.
+// that they cover the column); all loads are issued before the first LDS write.  A 128-byte line of
+// the layout is read by one wave, once: nontemporal, so that it does not push the partly written
+// lines of the results (16 bytes of each from this workgroup, the rest from its neighbours) out of
+// the L2 (64 fields of 2400x1200: y pass 725 -> 697 us; row-major columns, whose lines several
+// workgroups read, lose by it: 156 -> 203 us for 512x512x128).
 __device__ __forceinline__ void blocked_load_cols(const float *__restrict__ gv, const float *__restrict__ gw,
                                                   int64_t W, int64_t x0, int nl, int L, float *__restrict__ dv,
                                                   float *__restrict__ dw, int lstride)
@@ -883,8 +895,8 @@ __device__ __forceinline__ void blocked_load_cols(const float *__restrict__ gv, 
         const int r = r0 + k * rstep;
         if (r < L) {
             const int64_t o = blocked_index(r, x0 + 4 * q, W);
-            rv[k] = *reinterpret_cast<const float4 *>(gv + o);
-            rw[k] = *reinterpret_cast<const float4 *>(gw + o);
+            rv[k] = load_once(gv + o);
+            rw[k] = load_once(gw + o);
         }
     }
     float *a = dv + (4 * q) * lstride + r0, *b = dw + (4 * q) * lstride + r0;
@@ -934,7 +946,8 @@ __device__ __forceinline__ void blocked_store_cols(float *__restrict__ gv, float
 // into the v and w lines, instead of a separate pass writing them to HBM.  float32
 // arithmetic: the quotient with one Newton step, and f - offset as (f - hi) - lo with the
 // offset split into float32 hi + lo (f - hi is exact while f is within a factor 2 of hi).
-// float4 global loads when the rows allow.
+// float4 global loads when the rows allow, nontemporal: they are read once (the three passes of a
+// backward of 16 fields of 2400x1200 703 -> 674 us, the gather after them 73 -> 80).
 __device__ __forceinline__ void adjoint_ab(float fo, float go, float wv, float hi, float lo, float &a, float &b)
 {
     a = 0.f;
@@ -958,12 +971,10 @@ __device__ __forceinline__ void adjoint_load(const float *__restrict__ f, const 
     if ((L & 3) == 0 && (ls & 3) == 0 && aligned16(f) && aligned16(w) && aligned16(g)) {
         const int Lq = L >> 2;
         for (int l = 0; l < nl; ++l) {
-            const float4 *fl = reinterpret_cast<const float4 *>(f + l * ls);
-            const float4 *wl = reinterpret_cast<const float4 *>(w + l * ls);
-            const float4 *gl = reinterpret_cast<const float4 *>(g + l * ls);
             float *da = sa + l * lstride, *db = sb + l * lstride;
             for (int q = tid; q < Lq; q += nthr) {
-                const float4 fo = fl[q], go = gl[q], wv = wl[q];
+                const float4 fo = load_once(f + l * ls + 4 * q), go = load_once(g + l * ls + 4 * q),
+                             wv = load_once(w + l * ls + 4 * q);
                 float a, b;
                 adjoint_ab(fo.x, go.x, wv.x, hi, lo, a, b);
                 da[4 * q] = a;
@@ -1171,9 +1182,14 @@ __global__ __launch_bounds__(kFastBlock, 1) void k_fast_pass(
 {
     constexpr int kSegArr = SEG;
     extern __shared__ __align__(16) unsigned char smem[];
+    // The waves that fill their tile go first, those that filter it give way (64 fields of 2400x1200,
+    // us: x 640 -> 625, y 705 -> 685; the adjoint's passes of 16 fields 250 -> 235).  Not where columns
+    // are read in pieces of lines that other workgroups read too: y of 512x512x128 156 -> 161.
+    if (INJECT || adj_g) __builtin_amdgcn_s_setprio(2);
     const PassWork wk = work[blockIdx.x];
     const FieldDev &F = fields[wk.field];
     const PassField P = passes[wk.field];
+    if (P.blocked == kBlockedIn) __builtin_amdgcn_s_setprio(2);
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
     const int half = nthr >> 1;
@@ -1299,6 +1315,7 @@ __global__ __launch_bounds__(kFastBlock, 1) void k_fast_pass(
     // wave (lpl <= 64, a power of two; each field's half of the workgroup is whole waves),
     // else by workgroup barriers.  The tile IO after the loop spans all lines.
     float sb[kSegArr];
+    __builtin_amdgcn_s_setprio(0);
     for (int it = 0; it < niter; ++it) {
         const bool last = it + 1 == niter;
         const bool grp = (it + 1) % P.sgroup == 0;
