@@ -189,7 +189,7 @@ inline LineGeom line_geom(int64_t max_rect, int max_iter, int64_t max_len)
     return g;
 }
 
-// FP64 injection: one sorted entry's record (k_inject_records), in list order.
+// FP64 injection: one sorted entry's record (k_field_sort, k_inject_records), in list order.
 struct InjectRec {
     int x;              // base column
     uint32_t p;         // point index

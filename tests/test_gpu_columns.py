@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize('n', [40, 400])
 def test_columns(size, n):
     rng = np.random.default_rng(sum(size) + n)
-    dim, n = len(size), n
+    dim = len(size)
     pts = rng.uniform(-0.5, np.asarray(size) - 0.5, (n, dim))
     val = 10.0 + rng.normal(0.0, 2.0, n)
     field = dict(sigma=1.5, x0=np.zeros(dim), step=1.0, size=size, n=n, num_iter=4, max_dist=3.5)
