@@ -236,16 +236,24 @@ public:
         }
         stage_delete(b_);
     }
-    // host memory to the device, in stream order: through the block while it has room (src is free
-    // on return), else as a copy from src's own memory
+    hipStream_t stream() const { return s_; }
+    bool fits(size_t bytes) { return bytes <= kStageUp - used_ && block(); }
+    // the caller's arrays to the device, in stream order: through the block while it has room, else as
+    // a copy from src's own memory, which must stay until the stream's work is done
     hipError_t up(void *dst, const void *src, size_t bytes)
     {
         if (!bytes) return hipSuccess;
-        if (bytes > kStageUp - used_ || !block()) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s_);
+        if (!fits(bytes)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s_);
         char *const at = b_->p + used_;
         used_ += std::min(round_bytes(bytes), kStageUp - used_);
         std::memcpy(at, src, bytes);
         return hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, s_);
+    }
+    // The same for memory of the call's own (descriptors), which may go as soon as this returns: a
+    // synchronous copy where the block has no room.
+    hipError_t up_own(void *dst, const void *src, size_t bytes)
+    {
+        return fits(bytes) ? up(dst, src, bytes) : hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
     }
     // device memory to the host, after the work queued on the stream; complete on return
     hipError_t down(void *dst, const void *src, size_t bytes)
@@ -752,8 +760,8 @@ struct fb_plan {
     Stage *stage = nullptr;   // of the call that creates the plan, if it has one
 
     // several host arrays into one device block with one copy, each 256-byte aligned (a plan's
-    // descriptors and prefixes: one copy instead of one per array); without a stage the copy is
-    // synchronous
+    // descriptors and prefixes: one copy instead of one per array); without a stage, or with one whose
+    // block the points have filled, the copy is synchronous, since h goes on return
     struct Upload {
         void **dst;
         const void *src;
@@ -773,7 +781,7 @@ struct fb_plan {
             *u.dst = d + off;
             off += round_bytes(u.bytes ? u.bytes : 1);
         }
-        if (stage && total <= kStageUp / 2) FB_HIP_CHECK(stage->up(d, h.data(), total));
+        if (stage) FB_HIP_CHECK(stage->up_own(d, h.data(), total));
         else FB_HIP_CHECK(hipMemcpy(d, h.data(), total, hipMemcpyHostToDevice));
         return FB_OK;
     }
@@ -1882,7 +1890,7 @@ int fb_barnes(int method, int precision, int dim, int64_t n, const double *pts, 
         double *d_off, *d_out = (double *)out;
         if ((rc = sc.get(&d_f, 1)) || (rc = sc.get(&d_off, 1))) return rc;
         if (!on_dev && (rc = sc.get(&d_out, cells))) return rc;
-        FB_HIP_CHECK(stage.up(d_f, &F, sizeof(F)));
+        FB_HIP_CHECK(stage.up_own(d_f, &F, sizeof(F)));
         double *d_part;
         if ((rc = sc.get(&d_part, offsets_part_elems(1, n)))) return rc;
         if ((rc = launch_offsets(d_f, 1, n, d_val, d_part, d_off, s))) return rc;
@@ -2089,7 +2097,7 @@ int fb_barnes_s2(int method, int precision, int64_t n, const double *pts, const 
         double *d_off, *d_out = (double *)out;
         if ((rc = sc.get(&d_f, 1)) || (rc = sc.get(&d_off, 1))) return rc;
         if (!on_dev && (rc = sc.get(&d_out, cells))) return rc;
-        FB_HIP_CHECK(stage.up(d_f, &F, sizeof(F)));
+        FB_HIP_CHECK(stage.up_own(d_f, &F, sizeof(F)));
         double *d_part;
         if ((rc = sc.get(&d_part, offsets_part_elems(1, n)))) return rc;
         if ((rc = launch_offsets(d_f, 1, n, d_val, d_part, d_off, s))) return rc;
