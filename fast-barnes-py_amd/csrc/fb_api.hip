@@ -716,6 +716,7 @@ struct fb_plan {
         for (auto &u : uses)
             if (u.first == s) {
                 FB_HIP_CHECK(hipEventRecord(u.second, s));
+                if (s == up_stream) uploading = false;
                 return FB_OK;
             }
         hipEvent_t e = nullptr;
@@ -727,6 +728,7 @@ struct fb_plan {
             return FB_OK;
         }
         uses.push_back({s, e});
+        if (s == up_stream) uploading = false;
         return FB_OK;
     }
 
@@ -758,6 +760,10 @@ struct fb_plan {
         return FB_OK;
     }
     Stage *stage = nullptr;   // of the call that creates the plan, if it has one
+    // Staged uploads on up_stream that no recorded use covers yet: a plan that is given up before its
+    // run waits for them.
+    bool uploading = false;
+    hipStream_t up_stream = nullptr;
 
     // several host arrays into one device block with one copy, each 256-byte aligned (a plan's
     // descriptors and prefixes: one copy instead of one per array); without a stage, or with one whose
@@ -781,8 +787,11 @@ struct fb_plan {
             *u.dst = d + off;
             off += round_bytes(u.bytes ? u.bytes : 1);
         }
-        if (stage) FB_HIP_CHECK(stage->up_own(d, h.data(), total));
-        else FB_HIP_CHECK(hipMemcpy(d, h.data(), total, hipMemcpyHostToDevice));
+        if (stage) {
+            uploading = true;
+            up_stream = stage->stream();
+            FB_HIP_CHECK(stage->up_own(d, h.data(), total));
+        } else FB_HIP_CHECK(hipMemcpy(d, h.data(), total, hipMemcpyHostToDevice));
         return FB_OK;
     }
     template <class T>
@@ -795,7 +804,8 @@ struct fb_plan {
     }
     ~fb_plan()
     {
-        // kernels queued on a caller's stream may still read or write the buffers
+        // kernels or copies queued on a caller's stream may still read or write the buffers
+        if (uploading) (void)hipStreamSynchronize(up_stream);
         for (auto &u : uses) {
             (void)hipEventSynchronize(u.second);
             (void)hipEventDestroy(u.second);

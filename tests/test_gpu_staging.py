@@ -1,5 +1,7 @@
 """Single calls on host arrays (the pinned staging of fb_api.hip) give the bits of a plan on device
 buffers where the points leave the descriptors little room in the block's first megabyte, or none."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,27 @@ def test_points_fill_the_block(precision, size, n):
     got = interpolation.barnes(pts, val, precision=precision, **c)
     ref = BarnesBatch([dict(c, n=n)], precision=precision).interpolate([pts], [val])[0]
     assert _same(got, ref)
+
+
+def test_refused_calls_beside_good_ones():
+    """A call that is refused after its first upload (no FP32C line pass takes half kernels of 3000)
+    gives its blocks back while another thread's calls take blocks of the same sizes."""
+    pts, val, c = _field((300, 150), 3000, 1)
+    ref = BarnesBatch([dict(c, n=3000)], precision='fp32c').interpolate([pts], [val])[0]
+    bad = dict(c, sigma=6928.0, step=2.0, size=(16000, 40))
+    refused, good = [], []
+
+    def refuse():
+        for _ in range(50):
+            try:
+                interpolation.barnes(pts, val, precision='fp32c', **dict(bad, sigma=(6928.0, 4.0)))
+            except RuntimeError as e:
+                refused.append(str(e))
+
+    t = threading.Thread(target=refuse)
+    t.start()
+    for _ in range(50):
+        good.append(_same(interpolation.barnes(pts, val, precision='fp32c', **c), ref))
+    t.join()
+    assert len(refused) == 50 and all('fit no FP32C line pass' in e for e in refused)
+    assert all(good)
