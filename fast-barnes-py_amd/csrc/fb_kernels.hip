@@ -355,12 +355,12 @@ __global__ __launch_bounds__(kBlock) void k_inject_records(
 // 151x133x61 73 us, here 17; 24 fields of 3490 on 600x300 99 us, here 16.
 template <int DIM, bool ZEROED>
 __global__ __launch_bounds__(kBlock) void k_inject_cells(
-    const FieldDev *__restrict__ fields, int64_t npoints, const InjectRec *__restrict__ irec,
+    const FieldDev *__restrict__ fields, int64_t first, int64_t npoints, const InjectRec *__restrict__ irec,
     const uint32_t *__restrict__ row_start, const uint32_t *__restrict__ row_count, double *__restrict__ vg,
     double *__restrict__ wg)
 {
     constexpr int NC = 1 << DIM;
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (first + blockIdx.x) * kBlock + threadIdx.x;
     const uint32_t e = (uint32_t)(i >> DIM);
     if ((i >> DIM) >= npoints) return;
     const int own = (int)i & (NC - 1);
@@ -1892,23 +1892,17 @@ int launch_inject_cells(const FieldDev *d_fields, int64_t npoints, const InjectR
         set_error("FP64 injection: the plan has no record array");
         return FB_ERR_INVALID_ARGUMENT;
     }
-    const dim3 grid((unsigned)(((npoints << dim) + kBlock - 1) / kBlock)), block(kBlock);
-#define FB_CELLS(D_, Z_)                                                                                          \
-    hipLaunchKernelGGL((k_inject_cells<D_, Z_>), grid, block, 0, s, d_fields, npoints, d_irec, d_row_start, d_row_count, \
-                       d_vg, d_wg)
-    if (dim == 1) {
-        if (zeroed) FB_CELLS(1, true);
-        else FB_CELLS(1, false);
-    } else if (dim == 2) {
-        if (zeroed) FB_CELLS(2, true);
-        else FB_CELLS(2, false);
-    } else {
-        if (zeroed) FB_CELLS(3, true);
-        else FB_CELLS(3, false);
-    }
-#undef FB_CELLS
-    FB_HIP_CHECK(hipGetLastError());
-    return FB_OK;
+    return launch_parts(((npoints << dim) + kBlock - 1) / kBlock, kBlock, [&](int64_t first, unsigned count) {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(count), dim3(kBlock), 0, s, d_fields, first, npoints, d_irec, d_row_start,
+                               d_row_count, d_vg, d_wg);
+        };
+        if (dim == 1) zeroed ? launch(k_inject_cells<1, true>) : launch(k_inject_cells<1, false>);
+        else if (dim == 2) zeroed ? launch(k_inject_cells<2, true>) : launch(k_inject_cells<2, false>);
+        else zeroed ? launch(k_inject_cells<3, true>) : launch(k_inject_cells<3, false>);
+        FB_HIP_CHECK(hipGetLastError());
+        return FB_OK;
+    });
 }
 
 int launch_exact_lines(const FieldDev *d_fields, const int64_t *d_line_prefix, int nfields, int64_t nslots,

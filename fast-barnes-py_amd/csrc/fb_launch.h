@@ -2,9 +2,22 @@
 #pragma once
 
 #include "fastbarnes.h"
+#include <algorithm>
+
 #include "fb_internal.h"
 
 namespace fb {
+
+// A launch holds fewer than 2^32 work-items; larger grids run in parts.  launch(first, count) takes the
+// workgroups [first, first + count) of nwg and returns its status.
+template <class F>
+inline int launch_parts(int64_t nwg, int threads, F launch)
+{
+    const int64_t most = 0xFFFFFFFFll / threads;
+    for (int64_t first = 0; first < nwg; first += most)
+        if (const int rc = launch(first, (unsigned)std::min(most, nwg - first))) return rc;
+    return FB_OK;
+}
 
 // fb_sort.hip
 // The whole sort stage of fields of at most kLocalSortMax points and kLocalRowsMax x-lines, one
