@@ -55,6 +55,7 @@ struct StreamArgs {
     double *vg, *wg;
     const double *offsets;
     float *out;                 // last axis: the masked quotient goes here instead of vg, wg
+    int64_t wg0;                // first workgroup of the launch
 };
 
 // LDS position of (position, slot) of a block or ring: pairs of positions adjacent, so that a
@@ -159,7 +160,8 @@ __global__ __launch_bounds__(kLineWavesMax * 64) void k_exact_stream(StreamArgs 
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int f = find_seg(A.wg_prefix, A.nfields, blockIdx.x);
+    const int64_t b = A.wg0 + blockIdx.x;
+    const int f = find_seg(A.wg_prefix, A.nfields, b);
     const FieldDev &F = A.fields[f];
     const int nf = min(A.ni, F.num_iter - A.it0);
     if (nf <= 0) return;
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(kLineWavesMax * 64) void k_exact_stream(StreamArgs 
     const int64_t W = F.size[0], H = F.size[1], D = F.size[2];
     const int L = (int)F.size[axis];
     const int64_t nlines = axis == 0 ? H * D : axis == 1 ? W * D : W * H;
-    const int64_t l0 = ((int64_t)blockIdx.x - A.wg_prefix[f]) * HL;
+    const int64_t l0 = (b - A.wg_prefix[f]) * HL;
     const int nl = (int)min((int64_t)HL, nlines - l0);
     const int rect = A.rect_override > 0 ? A.rect_override : 2 * F.T[axis] + 1;
     const int h0 = (rect - 1) / 2, h1 = rect - h0;
@@ -342,13 +344,17 @@ int launch_exact_stream(const FieldDev *d_fields, const int64_t *d_wg_prefix, in
         set_error("FP64 lines: the kernel is too wide for the LDS rings");
         return FB_ERR_UNSUPPORTED;
     }
-    StreamArgs a{d_fields, d_wg_prefix, nfields, axis, rect_override, 0, g.ni, g.R, d_vg, d_wg, d_offsets, d_out};
-    for (int it0 = 0; it0 < max_iter; it0 += g.ni) {
-        a.it0 = it0;
-        const dim3 grid((unsigned)nwg), block(64 * ((g.ni + 64 / S - 1) / (64 / S) + 3));
-        if (axis == 0) hipLaunchKernelGGL(k_exact_stream<true>, grid, block, g.lds, s, a);
-        else hipLaunchKernelGGL(k_exact_stream<false>, grid, block, g.lds, s, a);
-        FB_HIP_CHECK(hipGetLastError());
+    StreamArgs a{d_fields, d_wg_prefix, nfields, axis, rect_override, 0, g.ni, g.R, d_vg, d_wg, d_offsets, d_out, 0};
+    const int threads = 64 * ((g.ni + 64 / S - 1) / (64 / S) + 3);
+    for (a.it0 = 0; a.it0 < max_iter; a.it0 += g.ni) {
+        const int rc = launch_parts(nwg, threads, [&](int64_t first, unsigned count) {
+            a.wg0 = first;
+            if (axis == 0) hipLaunchKernelGGL(k_exact_stream<true>, dim3(count), dim3(threads), g.lds, s, a);
+            else hipLaunchKernelGGL(k_exact_stream<false>, dim3(count), dim3(threads), g.lds, s, a);
+            FB_HIP_CHECK(hipGetLastError());
+            return FB_OK;
+        });
+        if (rc) return rc;
     }
     return FB_OK;
 }
