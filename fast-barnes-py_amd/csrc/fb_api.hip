@@ -1186,7 +1186,7 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     // walk them alone (5000 points on 100x90x60, 5400 rows: 86 us, the row buckets 28).
     P->local = P->max_n <= kLocalSortMax && P->max_rows <= kLocalRowsMax;
     const bool records = !fast;   // the FP64 injection reads its records, the FP32C x pass the list
-    TRY(P->alloc(&P->d_off_part, offsets_part_elems(nfields, P->max_n)));
+    TRY(P->alloc(&P->d_off_part, offsets_part_elems(nfields, P->npoints)));
     if (records) TRY(P->alloc(&P->d_irec, P->npoints));
     if (!P->local) {
         // keys, slots and composites are spent when the records are written and share their
@@ -1257,8 +1257,8 @@ int plan_sort(fb_plan *P, const double *pts, const double *val, bool raw, hipStr
                                  P->d_irec, {vg, wg}, s);
     // whole 16-byte words: the row counts' allocation is a multiple of 256 bytes
     const ZeroRange counts{(uint4 *)P->d_line_count, (P->nxlines + 3) / 4};
-    if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->max_n, val, P->d_off_part, P->d_done, {counts, vg, wg}, s)) ||
-        (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->max_n, P->npoints, pts, val, P->d_keys,
+    if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->npoints, val, P->d_off_part, P->d_done, {counts, vg, wg}, s)) ||
+        (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, pts, val, P->d_keys,
                                 P->d_line_count, P->d_slot, P->max_rows, P->d_rec, P->d_off_part, P->d_offsets, s)) ||
         (rc = row_bucket_sort(P->d_fields, P->d_pt_prefix, P->nfields, P->d_keys, P->d_slot, P->npoints,
                               P->d_line_start, P->d_line_count, P->nxlines, P->d_tiles, P->d_done, P->d_comp, P->d_list,
@@ -1537,7 +1537,7 @@ int fb_plan_backward(fb_plan *P, const double *d_pts, const double *d_val, const
                 return fail(FB_ERR_UNSUPPORTED, "the adjoint takes lines of at most the FP32C line pass's length "
                                                 "along y and z");
     hipStream_t s = (hipStream_t)stream;
-    int rc = launch_offsets(P->d_fields, P->nfields, P->max_n, d_val, P->d_off_part, P->d_offsets, s);
+    int rc = launch_offsets(P->d_fields, P->nfields, P->max_n, P->npoints, d_val, P->d_off_part, P->d_offsets, s);
     // the same scaled line passes; the first one forms a = g/W and b = -a(f - offset) in its tile
     // load, so a and b never round-trip through HBM
     for (int a = 0; a < P->dim && !rc; ++a)
@@ -1903,7 +1903,7 @@ int fb_barnes(int method, int precision, int dim, int64_t n, const double *pts, 
         FB_HIP_CHECK(stage.up_own(d_f, &F, sizeof(F)));
         double *d_part;
         if ((rc = sc.get(&d_part, offsets_part_elems(1, n)))) return rc;
-        if ((rc = launch_offsets(d_f, 1, n, d_val, d_part, d_off, s))) return rc;
+        if ((rc = launch_offsets(d_f, 1, n, n, d_val, d_part, d_off, s))) return rc;
         double r2 = 0.0;
         if (method == FB_METHOD_RADIUS) {
             // kdtree.prepare_search: radius**2 with radius = sqrt(-2 log(min_weight)) * sigma
@@ -2110,7 +2110,7 @@ int fb_barnes_s2(int method, int precision, int64_t n, const double *pts, const 
         FB_HIP_CHECK(stage.up_own(d_f, &F, sizeof(F)));
         double *d_part;
         if ((rc = sc.get(&d_part, offsets_part_elems(1, n)))) return rc;
-        if ((rc = launch_offsets(d_f, 1, n, d_val, d_part, d_off, s))) return rc;
+        if ((rc = launch_offsets(d_f, 1, n, n, d_val, d_part, d_off, s))) return rc;
         if ((rc = launch_naive_s2(d_pts, d_val, d_off, n, sigma[0], x0, step, size, d_out, s))) return rc;
         if (!on_dev) FB_HIP_CHECK(stage.down(out, d_out, cells * sizeof(double)));
         FB_HIP_CHECK(hipStreamSynchronize(s));

@@ -60,16 +60,27 @@ __global__ __launch_bounds__(kBlock) void k_offsets(const FieldDev *__restrict__
     if (threadIdx.x == 0) offsets[blockIdx.x] = field_offset(mn, mx, isn);
 }
 
-// The same over many workgroups per field (large fields): workgroup f*nchunk + c reduces chunk c
-// (kOffChunk values) of field f to (min, max, NaN flag); offsets_final combines a field's chunks.
+// The same over many workgroups per field (large fields): each reduces one chunk of kOffChunk values
+// to (min, max, NaN flag); offsets_final combines a field's chunks.  The chunks of field f begin at
+// workgroup pt_off / kOffChunk + f: at least as many as it has, and at most one more, so that one
+// large field among many small ones costs its own chunks only (4 million points beside 2000 fields of
+// 100, as many workgroups for each field as for the largest: sort stage 4.6 ms, now 0.37).
 constexpr int kOffChunk = 2048;     // values of a chunk
 constexpr int kOffSingle = 8192;    // fields of up to this many values: one workgroup each
 
-__device__ __forceinline__ void offsets_part(const FieldDev *__restrict__ fields, const double *__restrict__ val,
-                                             double *__restrict__ part, int64_t blk, int nchunk)
+__host__ __device__ inline int64_t first_chunk(int64_t pt_off, int64_t f) { return pt_off / kOffChunk + f; }
+
+__device__ __forceinline__ void offsets_part(const FieldDev *__restrict__ fields, int nfields,
+                                             const double *__restrict__ val, double *__restrict__ part, int64_t blk)
 {
-    const FieldDev &F = fields[blk / nchunk];
-    const int64_t b0 = (blk % nchunk) * kOffChunk;
+    int lo = 0, hi = nfields - 1;   // the last field that begins at blk or before
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (first_chunk(fields[mid].pt_off, mid) <= blk) lo = mid; else hi = mid - 1;
+    }
+    const FieldDev &F = fields[lo];
+    const int64_t b0 = (blk - first_chunk(F.pt_off, lo)) * kOffChunk;
+    if (b0 >= F.n) return;
     double mn = INFINITY, mx = -INFINITY;
     int isn = 0;
     minmax_range(val + F.pt_off, b0 + threadIdx.x, min(F.n, b0 + kOffChunk), kBlock, mn, mx, isn);
@@ -82,15 +93,17 @@ __device__ __forceinline__ void offsets_part(const FieldDev *__restrict__ fields
 }
 
 // One wave per field.
-__device__ __forceinline__ void offsets_final(const double *__restrict__ part, int nfields, int nchunk,
-                                              double *__restrict__ offsets, int64_t blk)
+__device__ __forceinline__ void offsets_final(const FieldDev *__restrict__ fields, int nfields,
+                                              const double *__restrict__ part, double *__restrict__ offsets,
+                                              int64_t blk)
 {
     const int64_t f = blk * (kBlock / 64) + (threadIdx.x >> 6);
     if (f >= nfields) return;
     double mn = INFINITY, mx = -INFINITY;
     int isn = 0;
-    for (int c = threadIdx.x & 63; c < nchunk; c += 64) {
-        const double *o = part + (f * nchunk + c) * 3;
+    const int64_t c0 = first_chunk(fields[f].pt_off, f), c1 = c0 + (fields[f].n + kOffChunk - 1) / kOffChunk;
+    for (int64_t c = c0 + (threadIdx.x & 63); c < c1; c += 64) {
+        const double *o = part + c * 3;
         mn = fmin(mn, o[0]);
         mx = fmax(mx, o[1]);
         if (o[2] != 0.0) isn = 1;
@@ -99,17 +112,17 @@ __device__ __forceinline__ void offsets_final(const double *__restrict__ part, i
     if ((threadIdx.x & 63) == 0) offsets[f] = field_offset(mn, mx, isn);
 }
 
-__global__ __launch_bounds__(kBlock) void k_offsets_part(const FieldDev *__restrict__ fields,
-                                                         const double *__restrict__ val, double *__restrict__ part,
-                                                         int nchunk)
+__global__ __launch_bounds__(kBlock) void k_offsets_part(const FieldDev *__restrict__ fields, int nfields,
+                                                         const double *__restrict__ val, double *__restrict__ part)
 {
-    offsets_part(fields, val, part, blockIdx.x, nchunk);
+    offsets_part(fields, nfields, val, part, blockIdx.x);
 }
 
-__global__ __launch_bounds__(kBlock) void k_offsets_final(const double *__restrict__ part, int nfields, int nchunk,
+__global__ __launch_bounds__(kBlock) void k_offsets_final(const FieldDev *__restrict__ fields, int nfields,
+                                                          const double *__restrict__ part,
                                                           double *__restrict__ offsets)
 {
-    offsets_final(part, nfields, nchunk, offsets, blockIdx.x);
+    offsets_final(fields, nfields, part, offsets, blockIdx.x);
 }
 
 // The first launch of the row-bucket sort stage: the offsets' chunks (the first noff workgroups) and
@@ -117,13 +130,13 @@ __global__ __launch_bounds__(kBlock) void k_offsets_final(const double *__restri
 // FP64 grids.
 constexpr int kZeroPer = 4;   // 16-byte stores of a thread
 
-__global__ __launch_bounds__(kBlock) void k_sort_begin(const FieldDev *__restrict__ fields,
+__global__ __launch_bounds__(kBlock) void k_sort_begin(const FieldDev *__restrict__ fields, int nfields,
                                                        const double *__restrict__ val, double *__restrict__ part,
-                                                       int nchunk, int64_t noff, uint32_t *__restrict__ done,
+                                                       int64_t noff, uint32_t *__restrict__ done,
                                                        ZeroRange z0, ZeroRange z1, ZeroRange z2)
 {
     if (blockIdx.x < noff) {
-        offsets_part(fields, val, part, blockIdx.x, nchunk);
+        offsets_part(fields, nfields, val, part, blockIdx.x);
         return;
     }
     int64_t b = blockIdx.x - noff;
@@ -154,11 +167,11 @@ __global__ __launch_bounds__(kBlock) void k_point_keys(const FieldDev *__restric
                                                        const double *__restrict__ val,
                                                        uint32_t *__restrict__ keys, uint32_t *__restrict__ row_count,
                                                        uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
-                                                       int64_t nkb, const double *__restrict__ part, int nchunk,
+                                                       int64_t nkb, const double *__restrict__ part,
                                                        double *__restrict__ offsets)
 {
     if (blockIdx.x >= nkb) {
-        offsets_final(part, nfields, nchunk, offsets, blockIdx.x - nkb);
+        offsets_final(fields, nfields, part, offsets, blockIdx.x - nkb);
         return;
     }
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -194,12 +207,12 @@ __global__ __launch_bounds__(kBlock) void k_point_keys_hist(const FieldDev *__re
                                                             uint32_t *__restrict__ keys,
                                                             uint32_t *__restrict__ row_count,
                                                             uint32_t *__restrict__ slot, PointRec *__restrict__ rec,
-                                                            int64_t nkb, const double *__restrict__ part, int nchunk,
+                                                            int64_t nkb, const double *__restrict__ part,
                                                             double *__restrict__ offsets)
 {
     extern __shared__ uint32_t hist[];   // nbins row counters (dynamic LDS)
     if (blockIdx.x >= nkb) {
-        offsets_final(part, nfields, nchunk, offsets, blockIdx.x - nkb);
+        offsets_final(fields, nfields, part, offsets, blockIdx.x - nkb);
         return;
     }
     __shared__ int64_t s_rbase;
@@ -1800,47 +1813,42 @@ inline unsigned nblocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock
 // ---------------------------------------------------------------------------
 // launchers
 
-int64_t offsets_part_elems(int nfields, int64_t max_n)
-{
-    return (int64_t)nfields * ((max_n + kOffChunk - 1) / kOffChunk) * 3;
-}
+int64_t offsets_part_elems(int nfields, int64_t npoints) { return 3 * first_chunk(npoints, nfields); }
 
-int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
-                   double *d_offsets, hipStream_t s)
+int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, int64_t npoints, const double *d_val,
+                   double *d_part, double *d_offsets, hipStream_t s)
 {
     if (!d_part || max_n <= kOffSingle) {
         hipLaunchKernelGGL(k_offsets, dim3(nfields), dim3(kBlock), 0, s, d_fields, d_val, d_offsets);
     } else {
-        const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
-        hipLaunchKernelGGL(k_offsets_part, dim3((unsigned)((int64_t)nchunk * nfields)), dim3(kBlock), 0, s, d_fields,
-                           d_val, d_part, nchunk);
+        hipLaunchKernelGGL(k_offsets_part, dim3((unsigned)first_chunk(npoints, nfields)), dim3(kBlock), 0, s, d_fields,
+                           nfields, d_val, d_part);
         FB_HIP_CHECK(hipGetLastError());
-        hipLaunchKernelGGL(k_offsets_final, dim3(nblocks((int64_t)nfields * 64)), dim3(kBlock), 0, s,
-                           (const double *)d_part, nfields, nchunk, d_offsets);
+        hipLaunchKernelGGL(k_offsets_final, dim3(nblocks((int64_t)nfields * 64)), dim3(kBlock), 0, s, d_fields,
+                           nfields, (const double *)d_part, d_offsets);
     }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
 
-int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
+int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t npoints, const double *d_val, double *d_part,
                       uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t s)
 {
-    const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
-    const int64_t noff = (int64_t)nchunk * nfields;
+    const int64_t noff = first_chunk(npoints, nfields);
     int64_t nz = 0;
     for (const ZeroRange &z : zero) nz += zero_blocks<kBlock, kZeroPer>(z);
     hipLaunchKernelGGL(k_sort_begin, dim3((unsigned)(noff + std::max<int64_t>(nz, 1))), dim3(kBlock), 0, s, d_fields,
-                       d_val, d_part, nchunk, noff, d_done, zero[0], zero[1], zero[2]);
+                       nfields, d_val, d_part, noff, d_done, zero[0], zero[1], zero[2]);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
 
-int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
-                      int64_t npoints, const double *d_pts, const double *d_val, uint32_t *d_keys,
-                      uint32_t *d_row_count, uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t s)
+int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
+                      const double *d_pts, const double *d_val, uint32_t *d_keys, uint32_t *d_row_count,
+                      uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets,
+                      hipStream_t s)
 {
     if (nfields <= 0) return FB_OK;
-    const int nchunk = (int)((max_n + kOffChunk - 1) / kOffChunk);
     const unsigned nfin = nblocks((int64_t)nfields * 64);
     // points per thread: enough for each workgroup to see many points per row, while keeping
     // at least ~512 workgroups; small point sets, and fields with more rows than the LDS
@@ -1855,12 +1863,11 @@ int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
         const int64_t per = ppt * kBlock, nkb = (npoints + per - 1) / per;
         hipLaunchKernelGGL(k_point_keys_hist, dim3((unsigned)(nkb + nfin)), dim3(kBlock), (size_t)nbins * 4, s,
                            d_fields, d_pt_prefix, nfields, npoints, (int)ppt, nbins, d_pts, d_val, d_keys, d_row_count, d_slot,
-                           d_rec, nkb, d_part, nchunk, d_offsets);
+                           d_rec, nkb, d_part, d_offsets);
     } else {
         const int64_t nkb = npoints > 0 ? nblocks(npoints) : 0;
         hipLaunchKernelGGL(k_point_keys, dim3((unsigned)(nkb + nfin)), dim3(kBlock), 0, s, d_fields, d_pt_prefix,
-                           nfields, npoints, d_pts, d_val, d_keys, d_row_count, d_slot, d_rec, nkb, d_part, nchunk,
-                           d_offsets);
+                           nfields, npoints, d_pts, d_val, d_keys, d_row_count, d_slot, d_rec, nkb, d_part, d_offsets);
     }
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;

@@ -42,19 +42,20 @@ int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nf
 // fb_kernels.hip -- injection front end
 // (min+max)/2 per field; with d_part (offsets_part_elems doubles) large fields are reduced
 // by many workgroups
-int64_t offsets_part_elems(int nfields, int64_t max_n);
-int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
-                   double *d_offsets, hipStream_t stream);
+int64_t offsets_part_elems(int nfields, int64_t npoints);
+int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, int64_t npoints, const double *d_val,
+                   double *d_part, double *d_offsets, hipStream_t stream);
 // The row buckets' first two launches.  launch_sort_begin: the offsets' chunks (d_part), *d_done = 0
 // and the ranges zeroed.  launch_point_keys: the offsets from the chunks; each point's base cell,
 // its base row's count (row = x-line index, integer atomics on zeroed counts) and its slot there.
 // max_rows: the most x-lines of any field.  d_rec (may be NULL): each in-grid point's PointRec, for
 // the FP32C injection
-int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t max_n, const double *d_val, double *d_part,
+int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t npoints, const double *d_val, double *d_part,
                       uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t stream);
-int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t max_n,
-                      int64_t npoints, const double *d_pts, const double *d_val, uint32_t *d_keys,
-                      uint32_t *d_row_count, uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets, hipStream_t stream);
+int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
+                      const double *d_pts, const double *d_val, uint32_t *d_keys, uint32_t *d_row_count,
+                      uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets,
+                      hipStream_t stream);
 
 // fb_kernels.hip -- FP64 path with the reference's operation order
 // Each sorted entry's FP64 injection record (row buckets).
