@@ -1153,6 +1153,12 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     for (int a = 0; a < 3; ++a) lslot[a].push_back(P->lslots[a]);
     for (int a = 0; a < P->dim && !fast; ++a) {
         P->lgeom[a] = line_geom(max_rect[a], P->max_iter, max_len[a]);
+        if (a && P->lgeom[a].ni) {
+            LineTimes t;
+            for (const FieldDev &d : P->fh)
+                t.add(P->lgeom[a], d.size[a], d.size[0] * d.size[1] * d.size[2] / d.size[a], d.T[a], d.num_iter);
+            if (!t.rings(P->lgeom[a])) P->lgeom[a] = LineGeom();
+        }
         const int64_t lines = P->lgeom[a].ni ? kLineSlots / 2 : 1;
         for (const FieldDev &d : P->fh) {
             lwg[a].push_back(P->lwgs[a]);
@@ -1215,9 +1221,9 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     } else if (!fast) {
         TRY(P->alloc(&P->d_vg, P->ncells));
         TRY(P->alloc(&P->d_wg, P->ncells));
-        bool wide = false;   // an axis for k_exact_lines, which needs the second pair of planes
-        for (int a = 0; a < P->dim; ++a) wide = wide || !P->lgeom[a].ni;
-        if (wide || arena) {   // the fixed scratch counts them always: its limit is one of sizes only
+        bool threads = false;   // an axis for k_exact_lines, which needs the second pair of planes
+        for (int a = 0; a < P->dim; ++a) threads = threads || !P->lgeom[a].ni;
+        if (threads || arena) {   // the fixed scratch counts them always: its limit is one of sizes only
             TRY(P->alloc(&P->d_vs, P->ncells));
             TRY(P->alloc(&P->d_ws, P->ncells));
         }
@@ -2313,7 +2319,12 @@ int fb_convolve_grid(int tail, int precision, int dim, const int64_t *size, cons
         if ((rc = fast_pass_init())) return rc;   // the line kernels' LDS limit
         for (int a = 0; a < dim; ++a) {
             // line slots, then the workgroups of k_exact_stream
-            const LineGeom g = line_geom(2 * (int64_t)F.T[a] + 1, num_iter, F.size[a]);
+            LineGeom g = line_geom(2 * (int64_t)F.T[a] + 1, num_iter, F.size[a]);
+            if (a && g.ni) {
+                LineTimes t;
+                t.add(g, F.size[a], nl[a], F.T[a], num_iter);
+                if (!t.rings(g)) g = LineGeom();
+            }
             const int64_t per = g.ni ? kLineSlots / 2 : 1, nwg = (nl[a] + per - 1) / per;
             const int64_t pre[4] = {0, 2 * nl[a], 0, nwg};
             FB_HIP_CHECK(hipMemcpy(d_pre, pre, sizeof(pre), hipMemcpyHostToDevice));

@@ -7,7 +7,8 @@
 //                   k_point_keys (cells and row counts), then the row buckets of fb_sort.hip
 //   FP64 path:      k_inject_cells, k_exact_stream (fb_lines.hip) along each axis, the last one
 //                   with the quotient -- the reference's operation order; k_exact_lines (one
-//                   thread per line) and k_exact_finalize for kernels too wide for the LDS
+//                   thread per line) and k_exact_finalize for kernels too wide for the LDS and
+//                   for short columns of large grids
 //   FP32C path:     k_fast_pass<inject> along x, k_fast_pass along y (and z);
 //                   quotient, offset and NaN mask fused into the last pass
 #include <algorithm>
