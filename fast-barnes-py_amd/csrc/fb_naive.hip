@@ -330,10 +330,14 @@ NaivePlan naive_plan(int dim, const int64_t *size, int64_t n)
 
 // Products need a few rows and columns to fill their tiles; fields of one axis or of fewer than 16
 // nodes along x or 16 rows run node by node (there is no more than an exponential per node and
-// station to save, and little work in all).
+// station to save, and little work in all).  So do few stations: node by node each takes 0.22 us, or 2 ps a
+// node where those fill the chip, and the products' further launches 38 us more than the one (64 stations on
+// 64x64 nodes 75 us a call, as products 105; 128 on 600x300 196 and 179, 16 on 1200x600 308 and 297).
 int64_t naive_work_elems(int radius, int dim, const int64_t *size, int64_t n)
 {
-    if (radius || dim < 2 || size[0] < 16 || size[1] * (dim == 3 ? size[2] : 1) < 16) return 0;
+    const int64_t rows = size[1] * (dim == 3 ? size[2] : 1);
+    if (radius || dim < 2 || size[0] < 16 || rows < 16) return 0;
+    if ((double)n * std::max(0.22, 2e-6 * (double)size[0] * (double)rows) < 38.0) return 0;
     const NaivePlan p = naive_plan(dim, size, n);
     if (p.ntiles * p.split > INT32_MAX) return 0;
     return p.kb * (p.wp + p.hp + p.dp + 1) + (p.parts ? 2 * p.split * p.plane : 0);

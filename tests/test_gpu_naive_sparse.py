@@ -51,3 +51,22 @@ def test_far_nodes_time():
     pts, val = _corner(3490, 4.0, 1)
     run = lambda size: interpolation.barnes(pts, val, 0.25, 0.0, 75.0 / size[0], size, method='naive')
     assert _best(lambda: run((600, 300)), 5) < 1.1 * _best(lambda: run((12000, 15)), 5)
+
+
+def test_few_stations_time():
+    """One station: one launch, as for as many nodes in 15 rows."""
+    pts, val = np.array([[20.0, 10.0]]), np.array([3.0])
+    run = lambda size: interpolation.barnes(pts, val, 5.0, 0.0, 1.0, size, method='naive')
+    assert _best(lambda: run((64, 64)), 30) < 1.25 * _best(lambda: run((273, 15)), 30)
+
+
+@pytest.mark.parametrize('size,n', [((17, 19), 172), ((17, 19), 173), ((65, 129), 179), ((600, 300), 105),
+                                    ((600, 300), 106), ((33, 40, 35), 181)])
+def test_both_sides_of_few(orc, size, n):
+    """No weight below exp(-2 * 3): 50 ulp of a weight's rounding and its products, as in
+    test_gpu_naive.py, are 1e-14 of the values' range."""
+    rng = np.random.default_rng(n)
+    pts, val = rng.uniform(0.0, 1.0, (n, len(size))) * np.asarray(size), rng.normal(3.0, 2.0, n)
+    out = interpolation.barnes(pts, val, 300.0, 0.0, 1.0, size, method='naive')
+    ref = orc.interpolate_naive(pts, val, np.full(len(size), 300.0), np.zeros(len(size)), np.ones(len(size)), size)
+    assert np.abs(out - ref).max() <= 1e-14 * np.ptp(val)
