@@ -7,6 +7,7 @@
 // result does not depend on timing.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "fb_internal.h"
 #include "fb_launch.h"
@@ -135,6 +136,8 @@ __device__ __forceinline__ void block_bitonic(unsigned long long *sk, int np2)
 // many as there may be points, keep the last step short: with one bucket per row (12 to 40 points) it
 // took 6 us more.  5001 points on 601x299: zero fill, keys with the offset and sort took 1.9 + 5.5 +
 // 15.6 us in launches of their own, this takes 14.8.
+//
+// THREADS (1024 or 256): a workgroup takes up to 8 points and 4 rows per thread with 8 buckets each.
 struct FieldSortArgs {
     const FieldDev *fields;
     const int64_t *pt_prefix;
@@ -147,17 +150,17 @@ struct FieldSortArgs {
     int nfields, np2, raw;   // np2: the LDS composites; raw: offset 0
 };
 
-constexpr int kBuckets = 8192;                                      // at least 2 * kLocalRowsMax
+constexpr int kSortPerThread = kLocalSortMax / kLocalSortThreads;   // points and buckets per thread
+constexpr int kRowsPerThread = kLocalRowsMax / kLocalSortThreads;   // rows: at most half as many
 constexpr int kRankMax = 64;                                        // largest bucket placed by rank
-constexpr int kSortPerThread = kLocalSortMax / kLocalSortThreads;   // points per thread
-constexpr int kBucketsPerThread = kBuckets / kLocalSortThreads;
-constexpr int kSortWaves = kLocalSortThreads / 64;
 constexpr int kSortZeroPer = 8;   // 16-byte stores of a zeroing thread
 constexpr int kRankStep = 4;      // LDS reads in flight of a rank; sk has as many entries to spare
 
-template <int DIM, bool EXACT>
-__global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs A)
+template <int DIM, bool EXACT, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_field_sort(FieldSortArgs A)
 {
+    constexpr int kBuckets = kSortPerThread * THREADS, kBucketsPerThread = kSortPerThread;
+    constexpr int kSortWaves = THREADS / 64;
     extern __shared__ __align__(16) unsigned char smem[];   // composites
     __shared__ __align__(16) uint32_t start[kBuckets + 4];  // the buckets' counts, then their starts
     __shared__ uint32_t wsum[kSortWaves], wmax[kSortWaves];
@@ -165,8 +168,8 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
     __shared__ int dnan[kSortWaves];
     if ((int64_t)blockIdx.x >= A.nfields) {
         int64_t b = (int64_t)blockIdx.x - A.nfields;
-        if (!zero_block<kLocalSortThreads, kSortZeroPer>(A.zero[0], b))
-            zero_block<kLocalSortThreads, kSortZeroPer>(A.zero[1], b);
+        if (!zero_block<THREADS, kSortZeroPer>(A.zero[0], b))
+            zero_block<THREADS, kSortZeroPer>(A.zero[1], b);
         return;
     }
     const int f = blockIdx.x, tid = threadIdx.x, wv = tid >> 6;
@@ -195,7 +198,7 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
         double c[kGroup][DIM];
 #pragma unroll
         for (int u = 0; u < kGroup; ++u) {
-            const int i = tid + (g + u) * kLocalSortThreads;
+            const int i = tid + (g + u) * THREADS;
             if (i < n) {
                 v[g + u] = A.val[p0 + i];
 #pragma unroll
@@ -205,12 +208,12 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
         if (g == 0) {
 #pragma unroll
             for (int q = 0; q < kBucketsPerThread / 4; ++q)
-                quads[tid + q * kLocalSortThreads] = make_uint4(0u, 0u, 0u, 0u);
+                quads[tid + q * THREADS] = make_uint4(0u, 0u, 0u, 0u);
             __syncthreads();
         }
 #pragma unroll
         for (int u = 0; u < kGroup; ++u) {
-            const int k = g + u, i = tid + k * kLocalSortThreads;
+            const int k = g + u, i = tid + k * THREADS;
             xi[k] = -1;
             if (i < n) {
                 if (v[k] != v[k]) isn = 1;
@@ -264,7 +267,7 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
 #pragma unroll
     for (int q = 0; q < kBucketsPerThread; q += 4)
         quads[tid * (kBucketsPerThread / 4) + q / 4] = make_uint4(rc[q], rc[q + 1], rc[q + 2], rc[q + 3]);
-    if (tid == kLocalSortThreads - 1) start[kBuckets] = run;
+    if (tid == THREADS - 1) start[kBuckets] = run;
 #pragma unroll
     for (int q = 0; q < kSortWaves; ++q) {
         big = max(big, wmax[q]);
@@ -275,25 +278,25 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
     const double off = A.raw ? 0.0 : field_offset(mn, mx, isn);
     if (tid == 0) A.offsets[f] = off;
     __syncthreads();
-    for (int r = tid; r < nr; r += kLocalSortThreads) {
+    for (int r = tid; r < nr; r += THREADS) {
         const uint32_t s0 = start[r << ls];
         A.row_start[F.xline_off + r] = dst + s0;
         A.row_count[F.xline_off + r] = start[(r + 1) << ls] - s0;
     }
     if constexpr (EXACT)
-        for (int i = (int)total + tid; i < n; i += kLocalSortThreads) A.irec[dst + i].row = kInvalidKey;
+        for (int i = (int)total + tid; i < n; i += THREADS) A.irec[dst + i].row = kInvalidKey;
 
     if (big <= (uint32_t)kRankMax) {
 #pragma unroll
         for (int k = 0; k < kSortPerThread; ++k)
             if (xi[k] >= 0)
                 sk[start[bs[k] & 0xffffu] + (bs[k] >> 16)] =
-                    ((unsigned long long)(uint32_t)xi[k] << 32) | (uint32_t)(p0 + tid + k * kLocalSortThreads);
+                    ((unsigned long long)(uint32_t)xi[k] << 32) | (uint32_t)(p0 + tid + k * THREADS);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < kSortPerThread; ++k) {
             if (xi[k] < 0) continue;
-            const uint32_t p = (uint32_t)(p0 + tid + k * kLocalSortThreads);
+            const uint32_t p = (uint32_t)(p0 + tid + k * THREADS);
             const unsigned long long e = ((unsigned long long)(uint32_t)xi[k] << 32) | p;
             const uint32_t b = bs[k] & 0xffffu, s0 = start[b], s1 = start[b + 1];
             uint32_t at = s0;
@@ -320,10 +323,10 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
     }
 
     const uint32_t W = (uint32_t)F.size[0];
-    for (int i = n + tid; i < A.np2; i += kLocalSortThreads) sk[i] = ~0ull;
+    for (int i = n + tid; i < A.np2; i += THREADS) sk[i] = ~0ull;
 #pragma unroll
     for (int k = 0; k < kSortPerThread; ++k) {
-        const int i = tid + k * kLocalSortThreads;
+        const int i = tid + k * THREADS;
         if (i < n)
             sk[i] = xi[k] < 0 ? ~0ull
                               : ((unsigned long long)(((bs[k] & 0xffffu) >> ls) * W + (uint32_t)xi[k]) << 32) |
@@ -331,7 +334,7 @@ __global__ __launch_bounds__(kLocalSortThreads) void k_field_sort(FieldSortArgs 
     }
     __syncthreads();
     block_bitonic(sk, A.np2);
-    for (int i = tid; i < (int)total; i += kLocalSortThreads) {
+    for (int i = tid; i < (int)total; i += THREADS) {
         const uint32_t p = (uint32_t)sk[i];
         if constexpr (EXACT) {
             PointPos pp;
@@ -569,9 +572,10 @@ int field_sort_init()
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {
         const int lds = (kLocalSortMax + kRankStep) * (int)sizeof(unsigned long long);
-        const void *fns[] = {(const void *)k_field_sort<1, false>, (const void *)k_field_sort<2, false>,
-                             (const void *)k_field_sort<3, false>, (const void *)k_field_sort<1, true>,
-                             (const void *)k_field_sort<2, true>,  (const void *)k_field_sort<3, true>,
+        constexpr int T = kLocalSortThreads;   // (the smaller workgroups' LDS needs no raised limit)
+        const void *fns[] = {(const void *)k_field_sort<1, false, T>, (const void *)k_field_sort<2, false, T>,
+                             (const void *)k_field_sort<3, false, T>, (const void *)k_field_sort<1, true, T>,
+                             (const void *)k_field_sort<2, true, T>,  (const void *)k_field_sort<3, true, T>,
                              (const void *)k_row_sort};
         for (const void *fn : fns)
             if (err == hipSuccess) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -599,21 +603,34 @@ int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
     while (np2 < max_n) np2 <<= 1;
     FieldSortArgs A{d_fields,   d_pt_prefix, d_pts, d_val,  d_offsets,          d_row_count, d_row_start,
                     d_out_vals, d_rec,       d_irec, {zero[0], zero[1]}, nfields, np2, raw ? 1 : 0};
-    int64_t grid = nfields;
-    for (const ZeroRange &z : zero) grid += zero_blocks<kLocalSortThreads, kSortZeroPer>(z);
     const size_t lds = (size_t)(np2 + kRankStep) * 8;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kLocalSortThreads), lds, stream, A);
+    auto launch = [&](auto kernel, int threads, int64_t zero_wgs) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(nfields + zero_wgs)), dim3(threads), lds, stream, A);
     };
-    if (d_irec) {
-        if (dim == 1) launch(k_field_sort<1, true>);
-        else if (dim == 2) launch(k_field_sort<2, true>);
-        else launch(k_field_sort<3, true>);
-    } else {
-        if (dim == 1) launch(k_field_sort<1, false>);
-        else if (dim == 2) launch(k_field_sort<2, false>);
-        else launch(k_field_sort<3, false>);
-    }
+    auto run = [&](auto threads) {
+        constexpr int T = decltype(threads)::value;
+        int64_t zero_wgs = 0;
+        for (const ZeroRange &z : zero) zero_wgs += zero_blocks<T, kSortZeroPer>(z);
+        if (d_irec) {
+            if (dim == 1) launch(k_field_sort<1, true, T>, T, zero_wgs);
+            else if (dim == 2) launch(k_field_sort<2, true, T>, T, zero_wgs);
+            else launch(k_field_sort<3, true, T>, T, zero_wgs);
+        } else {
+            if (dim == 1) launch(k_field_sort<1, false, T>, T, zero_wgs);
+            else if (dim == 2) launch(k_field_sort<2, false, T>, T, zero_wgs);
+            else launch(k_field_sort<3, false, T>, T, zero_wgs);
+        }
+    };
+    // One workgroup of 1024 threads runs on a CU at a time.  Fields of few rows and up to 1024 points are
+    // done as soon by 256 threads (1000 points on 60x40: one field 10.0 us of 1024 threads and 9.1 of 256, 200
+    // fields 13.4 and 12.6); up to 2048 points (one field of 2000 11.5 and 11.8 us) where there are more
+    // fields than CUs (300 fields 24.8 and 20.0).  2000 fields of 50 points on 30x20: 47.8 us of 1024
+    // threads, 14.3 of 256; zero fill, keys and sort in launches of their own took 31.5.
+    constexpr int kSmall = 256;
+    if (max_n <= kSmall * (nfields > 256 ? kSortPerThread : kSortPerThread / 2) && max_rows <= kSmall * kRowsPerThread)
+        run(std::integral_constant<int, kSmall>());
+    else
+        run(std::integral_constant<int, kLocalSortThreads>());
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }
