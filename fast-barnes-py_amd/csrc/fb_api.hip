@@ -674,8 +674,8 @@ struct fb_plan {
     bool local = false;     // k_field_sort takes the sort stage of every field; else row buckets
     uint32_t *d_list = nullptr;                                 // the sorted point list
     uint32_t *d_keys = nullptr, *d_slot = nullptr;              // row buckets: base cells, slots,
-    unsigned long long *d_comp = nullptr;                       // entries by row, scan tiles and counter
-    uint32_t *d_tiles = nullptr, *d_done = nullptr;
+    unsigned long long *d_comp = nullptr;                       // entries by row, scan tiles
+    uint32_t *d_tiles = nullptr;
     uint32_t *d_line_count = nullptr, *d_line_start = nullptr;
     PointRec *d_rec = nullptr;                  // FP32C: each point's position for the injection
     InjectRec *d_irec = nullptr;                // FP64: each sorted entry's injection record
@@ -1209,8 +1209,7 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
             TRY(P->alloc(&P->d_slot, P->npoints));
             P->d_list = P->d_keys;
         }
-        TRY(P->alloc(&P->d_tiles, scan_tiles(P->nxlines) + 1));
-        P->d_done = P->d_tiles + scan_tiles(P->nxlines);
+        TRY(P->alloc(&P->d_tiles, scan_tiles(P->nxlines)));
     } else if (!records) {
         TRY(P->alloc(&P->d_list, P->npoints));
     }
@@ -1263,12 +1262,11 @@ int plan_sort(fb_plan *P, const double *pts, const double *val, bool raw, hipStr
                                  P->d_irec, {vg, wg}, s);
     // whole 16-byte words: the row counts' allocation is a multiple of 256 bytes
     const ZeroRange counts{(uint4 *)P->d_line_count, (P->nxlines + 3) / 4};
-    if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->npoints, val, P->d_off_part, P->d_done, {counts, vg, wg}, s)) ||
+    if ((rc = launch_sort_begin(P->d_fields, P->nfields, P->npoints, val, P->d_off_part, {counts, vg, wg}, s)) ||
         (rc = launch_point_keys(P->d_fields, P->d_pt_prefix, P->nfields, P->npoints, pts, val, P->d_keys,
                                 P->d_line_count, P->d_slot, P->max_rows, P->d_rec, P->d_off_part, P->d_offsets, s)) ||
         (rc = row_bucket_sort(P->d_fields, P->d_pt_prefix, P->nfields, P->d_keys, P->d_slot, P->npoints,
-                              P->d_line_start, P->d_line_count, P->nxlines, P->d_tiles, P->d_done, P->d_comp, P->d_list,
-                              s)))
+                              P->d_line_start, P->d_line_count, P->nxlines, P->d_tiles, P->d_comp, P->d_list, s)))
         return rc;
     if (!P->d_irec) return FB_OK;
     if (raw && (rc = launch_zero(P->d_offsets, P->nfields * 8, s))) return rc;

@@ -127,21 +127,18 @@ __global__ __launch_bounds__(kBlock) void k_offsets_final(const FieldDev *__rest
 }
 
 // The first launch of the row-bucket sort stage: the offsets' chunks (the first noff workgroups) and
-// the zero fills, which do not depend on each other: the scan's counter `done`, the row counts and the
-// FP64 grids.
+// the zero fills, which do not depend on each other: the row counts and the FP64 grids.
 constexpr int kZeroPer = 4;   // 16-byte stores of a thread
 
 __global__ __launch_bounds__(kBlock) void k_sort_begin(const FieldDev *__restrict__ fields, int nfields,
                                                        const double *__restrict__ val, double *__restrict__ part,
-                                                       int64_t noff, uint32_t *__restrict__ done,
-                                                       ZeroRange z0, ZeroRange z1, ZeroRange z2)
+                                                       int64_t noff, ZeroRange z0, ZeroRange z1, ZeroRange z2)
 {
     if (blockIdx.x < noff) {
         offsets_part(fields, nfields, val, part, blockIdx.x);
         return;
     }
     int64_t b = blockIdx.x - noff;
-    if (b == 0 && threadIdx.x == 0) *done = 0u;
     if (zero_block<kBlock, kZeroPer>(z0, b) || zero_block<kBlock, kZeroPer>(z1, b)) return;
     zero_block<kBlock, kZeroPer>(z2, b);
 }
@@ -1833,13 +1830,13 @@ int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, int64_t
 }
 
 int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t npoints, const double *d_val, double *d_part,
-                      uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t s)
+                      const ZeroRange (&zero)[3], hipStream_t s)
 {
     const int64_t noff = first_chunk(npoints, nfields);
     int64_t nz = 0;
     for (const ZeroRange &z : zero) nz += zero_blocks<kBlock, kZeroPer>(z);
     hipLaunchKernelGGL(k_sort_begin, dim3((unsigned)(noff + std::max<int64_t>(nz, 1))), dim3(kBlock), 0, s, d_fields,
-                       nfields, d_val, d_part, noff, d_done, zero[0], zero[1], zero[2]);
+                       nfields, d_val, d_part, noff, zero[0], zero[1], zero[2]);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
 }

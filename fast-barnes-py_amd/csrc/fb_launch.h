@@ -31,13 +31,12 @@ int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
                       uint32_t *d_row_count, uint32_t *d_row_start, uint32_t *d_out_vals, PointRec *d_rec,
                       InjectRec *d_irec, const ZeroRange (&zero)[2], hipStream_t stream);
 // fb_sort.hip -- row buckets for all other plans: the row starts from the row counts (scan_tiles(nrows)
-// words of d_tiles and the zeroed counter d_done), the in-grid points into their rows (d_comp), each
+// words of d_tiles), the in-grid points into their rows (d_comp), each
 // row sorted by (key, point index) into d_list, which may be d_keys' memory.
 int64_t scan_tiles(int64_t n);
 int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, const uint32_t *d_keys,
                     const uint32_t *d_slot, int64_t npoints, uint32_t *d_row_start, const uint32_t *d_row_count,
-                    int64_t nrows, uint32_t *d_tiles, uint32_t *d_done, unsigned long long *d_comp, uint32_t *d_list,
-                    hipStream_t stream);
+                    int64_t nrows, uint32_t *d_tiles, unsigned long long *d_comp, uint32_t *d_list, hipStream_t stream);
 
 // fb_kernels.hip -- injection front end
 // (min+max)/2 per field; with d_part (offsets_part_elems doubles) large fields are reduced
@@ -45,13 +44,13 @@ int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nf
 int64_t offsets_part_elems(int nfields, int64_t npoints);
 int launch_offsets(const FieldDev *d_fields, int nfields, int64_t max_n, int64_t npoints, const double *d_val,
                    double *d_part, double *d_offsets, hipStream_t stream);
-// The row buckets' first two launches.  launch_sort_begin: the offsets' chunks (d_part), *d_done = 0
-// and the ranges zeroed.  launch_point_keys: the offsets from the chunks; each point's base cell,
+// The row buckets' first two launches.  launch_sort_begin: the offsets' chunks (d_part) and the ranges
+// zeroed.  launch_point_keys: the offsets from the chunks; each point's base cell,
 // its base row's count (row = x-line index, integer atomics on zeroed counts) and its slot there.
 // max_rows: the most x-lines of any field.  d_rec (may be NULL): each in-grid point's PointRec, for
 // the FP32C injection
 int launch_sort_begin(const FieldDev *d_fields, int nfields, int64_t npoints, const double *d_val, double *d_part,
-                      uint32_t *d_done, const ZeroRange (&zero)[3], hipStream_t stream);
+                      const ZeroRange (&zero)[3], hipStream_t stream);
 int launch_point_keys(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, int64_t npoints,
                       const double *d_pts, const double *d_val, uint32_t *d_keys, uint32_t *d_row_count,
                       uint32_t *d_slot, int64_t max_rows, PointRec *d_rec, const double *d_part, double *d_offsets,

@@ -48,14 +48,14 @@ __device__ __forceinline__ uint32_t block_before(uint32_t v, uint32_t *wsum, uin
 
 // ---- scan ----------------------------------------------------------------
 
-// out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of all tiles
-// before tile t, formed by the workgroup that ends last (no workgroup waits for another).
+// out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of tile t (a single
+// tile: 0); k_scan_sums then makes that the sum of all tiles before tile t.  (In one launch, the workgroup
+// that ends last taking the sums, each workgroup's release before its count writes back its L2: 50 ns a tile,
+// 98 us for 2 million rows and 10.9 for 200 thousand; two launches take 9.1 and 5.6.)
 __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-                                                         int64_t n, uint32_t *__restrict__ tiles,
-                                                         uint32_t *__restrict__ done)
+                                                         int64_t n, uint32_t *__restrict__ tiles)
 {
     __shared__ uint32_t wsum[kThreads / 64];
-    __shared__ uint32_t last;
     const int tid = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)tid * kItems;
     uint32_t v[kItems] = {}, sum = 0, total;
@@ -74,18 +74,30 @@ __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restr
         if (base + i < n) out[base + i] = run;
         run += v[i];
     }
-    if (tid == 0) {
-        __hip_atomic_store(&tiles[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
+    if (tid == 0) tiles[blockIdx.x] = gridDim.x > 1 ? total : 0u;
+}
+
+constexpr int kSumThreads = 1024;
+
+// The exclusive scan of the tiles' sums in place, by one workgroup, kSumThreads * kItems of them a round.
+__global__ __launch_bounds__(kSumThreads) void k_scan_sums(uint32_t *__restrict__ tiles, int64_t n)
+{
+    __shared__ uint32_t wsum[kSumThreads / 64];
     uint32_t carry = 0;
-    for (int64_t t0 = 0; t0 < gridDim.x; t0 += kThreads) {
-        const int64_t t = t0 + tid;
-        const uint32_t x = t < gridDim.x ? __hip_atomic_load(&tiles[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-        const uint32_t before = block_before(x, wsum, total);
-        if (t < gridDim.x) tiles[t] = carry + before;
+    for (int64_t t0 = 0; t0 < n; t0 += kSumThreads * kItems) {
+        const int64_t base = t0 + (int64_t)threadIdx.x * kItems;
+        uint32_t v[kItems], sum = 0, total;
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            v[i] = base + i < n ? tiles[base + i] : 0u;
+            sum += v[i];
+        }
+        uint32_t run = carry + block_before(sum, wsum, total);
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            if (base + i < n) tiles[base + i] = run;
+            run += v[i];
+        }
         carry += total;
         __syncthreads();   // wsum is rewritten
     }
@@ -438,8 +450,10 @@ __device__ __forceinline__ void rank_row(const unsigned long long *__restrict__ 
     }
 }
 
-// The rows of workgroup b are b, b + gridDim.x, ...: neighbouring rows, which tend to be of a
-// size, go to different workgroups.  A thread completes its row's start and sorts it if it is
+// The rows of workgroup b are the groups b, b + gridDim.x, ... of 1 << shift rows: neighbouring rows, which tend
+// to be of a size, go to different workgroups, one by one while a workgroup's threads take all of its rows at
+// once, else 16 by 16, so that a wave reads whole 64-byte pieces of the counts and starts (2 million rows
+// 40 -> 13 us).  A thread completes its row's start and sorts it if it is
 // small; the workgroup's waves then take its rows of up to kRowWave entries, each wave in its own
 // slice of the LDS, by rank or by the bitonic network (within one wave every step only needs its LDS
 // operations complete: a wavefront fence, never a barrier); then the whole workgroup its larger rows:
@@ -450,7 +464,8 @@ __device__ __forceinline__ void rank_row(const unsigned long long *__restrict__ 
 // of rows for each kind) and the composites in one 64-bit array instead of two of 32: 16 fields of
 // 2400x1200 (19200 rows, 1.6 million points), scatter 25 + sorts 40 us, now 21 + 32; 65536 rows of 3 points
 // 7.1 + 14.3 us, now 6.2 + 9.0.  Of 512 threads with slices of 1024 composites it took 41 and 8.9.
-__global__ __launch_bounds__(kRowThreads) void k_row_sort(int64_t nrows, const uint32_t *__restrict__ row_count,
+__global__ __launch_bounds__(kRowThreads) void k_row_sort(int64_t nrows, int shift,
+                                                          const uint32_t *__restrict__ row_count,
                                                           uint32_t *__restrict__ row_start,
                                                           const uint32_t *__restrict__ tiles,
                                                           const unsigned long long *__restrict__ comp,
@@ -463,7 +478,8 @@ __global__ __launch_bounds__(kRowThreads) void k_row_sort(int64_t nrows, const u
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     unsigned long long *const sk = skb + wv * kRowWave;
     for (int64_t q0 = 0; q0 * gridDim.x < nrows; q0 += kRowThreads) {
-        const int64_t r = blockIdx.x + (q0 + tid) * gridDim.x;
+        const int64_t q = q0 + tid;
+        const int64_t r = ((blockIdx.x + (q >> shift) * gridDim.x) << shift) + (q & ((1 << shift) - 1));
         if (tid < 2) s_count[tid] = 0u;
         __syncthreads();
         uint32_t n = 0, s0 = 0;
@@ -546,21 +562,25 @@ int64_t scan_tiles(int64_t n) { return n > 0 ? cdiv(n, kTile) : 1; }
 
 int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nfields, const uint32_t *d_keys,
                     const uint32_t *d_slot, int64_t npoints, uint32_t *d_row_start, const uint32_t *d_row_count,
-                    int64_t nrows, uint32_t *d_tiles, uint32_t *d_done, unsigned long long *d_comp, uint32_t *d_list,
-                    hipStream_t stream)
+                    int64_t nrows, uint32_t *d_tiles, unsigned long long *d_comp, uint32_t *d_list, hipStream_t stream)
 {
     if (nrows <= 0) return FB_OK;
     hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)scan_tiles(nrows)), dim3(kThreads), 0, stream, d_row_count,
-                       d_row_start, nrows, d_tiles, d_done);
+                       d_row_start, nrows, d_tiles);
     FB_HIP_CHECK(hipGetLastError());
+    if (scan_tiles(nrows) > 1) {
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumThreads), 0, stream, d_tiles, scan_tiles(nrows));
+        FB_HIP_CHECK(hipGetLastError());
+    }
     if (npoints > 0) {
         hipLaunchKernelGGL(k_row_scatter, dim3((unsigned)cdiv(npoints, kThreads)), dim3(kThreads), 0, stream, d_fields,
                            d_pt_prefix, nfields, npoints, d_keys, d_slot, (const uint32_t *)d_row_start,
                            (const uint32_t *)d_tiles, d_comp);
         FB_HIP_CHECK(hipGetLastError());
     }
+    const int shift = nrows > (int64_t)kRowGrid * kRowThreads ? 4 : 0;
     hipLaunchKernelGGL(k_row_sort, dim3((unsigned)std::min<int64_t>(nrows, kRowGrid)), dim3(kRowThreads),
-                       (size_t)kLocalSortMax * sizeof(unsigned long long), stream, nrows, d_row_count, d_row_start,
+                       (size_t)kLocalSortMax * sizeof(unsigned long long), stream, nrows, shift, d_row_count, d_row_start,
                        (const uint32_t *)d_tiles, (const unsigned long long *)d_comp, d_list);
     FB_HIP_CHECK(hipGetLastError());
     return FB_OK;
