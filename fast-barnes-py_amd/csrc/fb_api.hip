@@ -1188,9 +1188,12 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
         P->max_n = std::max(P->max_n, d.n);
         P->max_rows = std::max(P->max_rows, d.size[1] * d.size[2]);
     }
-    // One workgroup per field sorts fields of few points and rows; beyond, a workgroup per field would
-    // walk them alone (5000 points on 100x90x60, 5400 rows: 86 us, the row buckets 28).
-    P->local = P->max_n <= kLocalSortMax && P->max_rows <= kLocalRowsMax;
+    // One workgroup per field sorts fields of up to 8192 points and 4096 rows, or 2048 points and 8192 rows:
+    // many rows cost it little (40 fields of 5000 rows and 8 points 11 us, by row buckets 32), but leave a
+    // bucket to a row, and many points in few of those rows go to its bitonic network (5000 points in 100 of
+    // 5000 rows 75 us, by row buckets 26; 2000 points 14 and 23).
+    P->local = P->max_n <= kLocalSortMax && P->max_rows <= kLocalRowsMax &&
+               (P->max_rows <= kLocalRowsMax / 2 || P->max_n <= kLocalSortMax / 4);
     const bool records = !fast;   // the FP64 injection reads its records, the FP32C x pass the list
     TRY(P->alloc(&P->d_off_part, offsets_part_elems(nfields, P->npoints)));
     if (records) TRY(P->alloc(&P->d_irec, P->npoints));

@@ -13,7 +13,7 @@ namespace fb {
 constexpr uint32_t kInvalidKey = 0xFFFFFFFFu;
 // largest field (points, x-lines) the per-field LDS sort takes (64-bit entries: 64 KiB of LDS)
 constexpr int kLocalSortMax = 8192;
-constexpr int kLocalRowsMax = 4096;
+constexpr int kLocalRowsMax = 8192;
 
 // 16-byte words from p on that a kernel zeroes
 struct ZeroRange {

@@ -149,7 +149,7 @@ __device__ __forceinline__ void block_bitonic(unsigned long long *sk, int np2)
 // took 6 us more.  5001 points on 601x299: zero fill, keys with the offset and sort took 1.9 + 5.5 +
 // 15.6 us in launches of their own, this takes 14.8.
 //
-// THREADS (1024 or 256): a workgroup takes up to 8 points and 4 rows per thread with 8 buckets each.
+// THREADS (1024 or 256): a workgroup takes up to 8 points and 8 rows per thread and has as many buckets.
 struct FieldSortArgs {
     const FieldDev *fields;
     const int64_t *pt_prefix;
@@ -162,8 +162,8 @@ struct FieldSortArgs {
     int nfields, np2, raw;   // np2: the LDS composites; raw: offset 0
 };
 
-constexpr int kSortPerThread = kLocalSortMax / kLocalSortThreads;   // points and buckets per thread
-constexpr int kRowsPerThread = kLocalRowsMax / kLocalSortThreads;   // rows: at most half as many
+constexpr int kSortPerThread = kLocalSortMax / kLocalSortThreads;   // points, rows and buckets per thread
+static_assert(kLocalRowsMax <= kLocalSortMax, "a row has at least one bucket");
 constexpr int kRankMax = 64;                                        // largest bucket placed by rank
 constexpr int kSortZeroPer = 8;   // 16-byte stores of a zeroing thread
 constexpr int kRankStep = 4;      // LDS reads in flight of a rank; sk has as many entries to spare
@@ -647,7 +647,7 @@ int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
     // fields than CUs (300 fields 24.8 and 20.0).  2000 fields of 50 points on 30x20: 47.8 us of 1024
     // threads, 14.3 of 256; zero fill, keys and sort in launches of their own took 31.5.
     constexpr int kSmall = 256;
-    if (max_n <= kSmall * (nfields > 256 ? kSortPerThread : kSortPerThread / 2) && max_rows <= kSmall * kRowsPerThread)
+    if (max_n <= kSmall * (nfields > 256 ? kSortPerThread : kSortPerThread / 2) && max_rows <= kSmall * kSortPerThread)
         run(std::integral_constant<int, kSmall>());
     else
         run(std::integral_constant<int, kLocalSortThreads>());

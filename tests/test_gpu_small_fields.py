@@ -22,12 +22,12 @@ def _bits(a):
     return np.where(np.isnan(a), np.float32(0), a).view(np.uint32), np.isnan(a)
 
 
-# points around the limits of a thread's share, rows around 1024 (1025: 1024 threads for every field)
+# points around the limits of a thread's share, rows around 2048 (2049: 1024 threads for every field)
 @pytest.mark.parametrize('precision', ['fp32c', 'fp64'])
 @pytest.mark.parametrize('size,n,hot', [((20, 30), 1, False), ((20, 30), 255, False), ((20, 30), 1024, False),
                                         ((20, 30), 1025, False), ((20, 30), 2048, False), ((20, 30), 2049, False),
                                         ((20, 30), 2047, True), ((300,), 900, True), ((300,), 2048, False),
-                                        ((14, 1024), 700, False), ((14, 1025), 700, False),
+                                        ((14, 2048), 700, False), ((14, 2049), 700, False),
                                         ((14, 13, 12), 1500, False), ((14, 13, 12), 300, True)])
 def test_small_fields_bitwise(precision, size, n, hot):
     rng = np.random.default_rng(n)
