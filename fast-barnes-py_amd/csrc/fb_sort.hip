@@ -48,17 +48,30 @@ __device__ __forceinline__ uint32_t block_before(uint32_t v, uint32_t *wsum, uin
 
 // ---- scan ----------------------------------------------------------------
 
-// out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of tile t (a single
-// tile: 0); k_scan_sums then makes that the sum of all tiles before tile t.  (In one launch, the workgroup
-// that ends last taking the sums, each workgroup's release before its count writes back its L2: 50 ns a tile,
-// 98 us for 2 million rows and 10.9 for 200 thousand; two launches take 9.1 and 5.6.)
+// out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of all tiles before tile
+// t: up to kFewTiles tiles each workgroup sums the words before its own, which spares a launch; beyond that
+// tiles[t] is left the sum of tile t, which k_scan_sums makes it of.  (In one launch, the workgroup that ends
+// last taking the sums, each workgroup's release before its count writes back its L2: 50 ns a tile, 98 us
+// for 2 million rows and 10.9 for 200 thousand; two launches take 9.1 and 5.6.)
+constexpr int kFewTiles = 16;
+
 __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
                                                          int64_t n, uint32_t *__restrict__ tiles)
 {
-    __shared__ uint32_t wsum[kThreads / 64];
+    __shared__ uint32_t wsum[kThreads / 64], wpre[kThreads / 64];
     const int tid = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)tid * kItems;
-    uint32_t v[kItems] = {}, sum = 0, total;
+    uint32_t v[kItems] = {}, sum = 0, total, before = 0;
+    const bool few = gridDim.x <= kFewTiles;
+    if (few) {
+        uint32_t pre = 0;
+#pragma unroll 4
+        for (int t = 0; t < (int)blockIdx.x; ++t) {
+            const uint4 x = reinterpret_cast<const uint4 *>(in + (int64_t)t * kTile)[tid];
+            pre += x.x + x.y + x.z + x.w;
+        }
+        block_before(pre, wpre, before);
+    }
     if (base + kItems <= n) {
         const uint4 x = *reinterpret_cast<const uint4 *>(in + base);
         v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
@@ -74,8 +87,10 @@ __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restr
         if (base + i < n) out[base + i] = run;
         run += v[i];
     }
-    if (tid == 0) tiles[blockIdx.x] = gridDim.x > 1 ? total : 0u;
+    if (tid == 0) tiles[blockIdx.x] = few ? before : total;
 }
+
+static_assert(kTile == kThreads * 4, "a thread reads 16 bytes of a tile");
 
 constexpr int kSumThreads = 1024;
 
@@ -568,7 +583,7 @@ int row_bucket_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int nf
     hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)scan_tiles(nrows)), dim3(kThreads), 0, stream, d_row_count,
                        d_row_start, nrows, d_tiles);
     FB_HIP_CHECK(hipGetLastError());
-    if (scan_tiles(nrows) > 1) {
+    if (scan_tiles(nrows) > kFewTiles) {
         hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumThreads), 0, stream, d_tiles, scan_tiles(nrows));
         FB_HIP_CHECK(hipGetLastError());
     }
