@@ -195,6 +195,7 @@ struct StageBlock {
 };
 
 struct StagePool {
+    StagePool() { idle.reserve(kStageKeep); }   // a block is given back without allocating
     std::mutex mu;
     std::vector<StageBlock *> idle;
 };

@@ -57,3 +57,36 @@ def test_refused_calls_beside_good_ones():
     t.join()
     assert len(refused) == 50 and all('fit no FP32C line pass' in e for e in refused)
     assert all(good)
+
+
+@pytest.mark.parametrize('size,method', [((2600, 1700), 'optimized_convolution'), ((4099, 2053), 'convolution'),
+                                         ((2048, 2048), 'optimized_convolution')])
+def test_results_of_several_rounds(size, method):
+    """Results of more than the 16 MB of the block's slots come down in rounds (16 MB exactly: in one)."""
+    pts, val, c = _field(size, 3000, size[0])
+    got = interpolation.barnes(pts, val, method=method, **c)
+    ref = BarnesBatch([dict(c, n=3000, method=method)], precision='fp64').interpolate([pts], [val])[0]
+    assert _same(got, ref)
+
+
+def test_concurrent_callers():
+    """More callers at once than idle blocks are kept, with results of one slot and of several."""
+    sizes = [(300, 150), (1200, 600), (2400, 1200), (600, 300)]
+    cases = []
+    for k, size in enumerate(sizes):
+        pts, val, c = _field(size, 2000 + 500 * k, k)
+        ref = BarnesBatch([dict(c, n=len(val))], precision='fp64').interpolate([pts], [val])[0]
+        cases.append((pts, val, c, ref))
+    good = [0] * len(cases)
+
+    def call(k):
+        pts, val, c, ref = cases[k]
+        for _ in range(12):
+            good[k] += _same(interpolation.barnes(pts, val, **c), ref)
+
+    threads = [threading.Thread(target=call, args=(k,)) for k in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert good == [12] * len(cases)
