@@ -73,7 +73,7 @@ int launch_inject_cells(const FieldDev *d_fields, int64_t npoints, const InjectR
 int launch_exact_lines(const FieldDev *d_fields, const int64_t *d_line_prefix, int nfields, int64_t nslots,
                        int axis, int rect_len, double *d_vg, double *d_wg, double *d_vs, double *d_ws,
                        hipStream_t stream);
-// fb_lines.hip -- FP64 lines through LDS rings, every iteration a wave (k_exact_stream), the same
+// fb_lines.hip -- FP64 lines through LDS rings, all iterations at once (k_exact_stream), the same
 // bits as launch_exact_lines: d_wg_prefix[f] = first workgroup of field f (ceil(lines / (kLineSlots/2))
 // each, nwg in all), g = line_geom of the fields' widest kernel (2T+1 or rect_override) and
 // max_iter = their most iterations.  d_out (last axis, may be NULL): the masked quotient is

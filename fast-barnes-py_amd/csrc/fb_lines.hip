@@ -4,9 +4,9 @@
 // _accumulate_tail_array (interpolation.py:484-533) runs num_iter iterations over a line, each a
 // running sum: step k adds in[k+h0], subtracts in[k-h1] and writes the sum plus alpha times the
 // two tail terms.  Iteration i's step k needs iteration i-1 only up to k+h0+1, so the iterations
-// of one line overlap in time: k_exact_stream gives every iteration a wave of its own, and the
-// waves pass blocks of kLineStep outputs through LDS rings, each wave h0/kLineStep + 2 blocks
-// behind the one before it.  Every running sum still adds its terms in the reference's order, so
+// of one line overlap in time: k_exact_stream gives every iteration lanes of its own, four iterations
+// of 16 slots to a wave, and they pass blocks of kLineStep outputs through LDS rings, each iteration
+// h0/kLineStep + 2 blocks behind the one before it.  Every running sum still adds its terms in the reference's order, so
 // the results are the reference's bits; the line's chain of dependent steps is num_iter times
 // shorter, and the grids are read and written once per pass instead of once per iteration.
 //
@@ -83,7 +83,7 @@ __device__ __forceinline__ void read_terms(const double *in, int from, double (&
 struct IterLane {
     const double *in;     // ring read, at the lane's slot
     double *out;          // ring or output blocks written, at the lane's slot
-    int h0, h1, L, NT;
+    int h0, h1, L;
     int lag, qend;        // first tick, end of the blocks it writes
     int ticks, R;
     int nout;             // blocks of the output ring (2: the output blocks, which have no mirror)
@@ -259,7 +259,6 @@ __global__ __launch_bounds__(kLineWavesMax * 64) void k_exact_stream(StreamArgs 
         I.h0 = h0;
         I.h1 = h1;
         I.L = L;
-        I.NT = NT;
         I.lag = i * (d + 1);
         I.qend = i > nf ? 0 : to_ring ? NT + d : NT;   // the next iteration reads d blocks past the line
         I.ticks = ticks;
