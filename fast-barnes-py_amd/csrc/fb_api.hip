@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "fb_launch.h"
+#include "fb_line_choice.h"
 
 // Workspace of fb_barnes_noalloc, reserved with the code object on every device the library
 // runs on.  Host code uses the per-device address noalloc_scratch() returns, never this name.
@@ -1113,7 +1114,6 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     const int fast = precision == FB_PREC_FP32C;
     P->fh.resize(nfields);
     std::vector<int64_t> pt_prefix, xline_prefix, cell_prefix, lslot[3], lwg[3];
-    int64_t max_rect[3] = {1, 1, 1}, max_len[3] = {1, 1, 1};
     for (int f = 0; f < nfields; ++f) {
         int rc = make_field(fields[f], P->fh[f], fast);
         if (rc) { delete P; return rc; }
@@ -1134,10 +1134,6 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
             lslot[a].push_back(P->lslots[a]);
             if (a < P->dim) P->lslots[a] += 2 * nl[a];
         }
-        for (int a = 0; a < 3; ++a) {
-            max_rect[a] = std::max(max_rect[a], 2 * (int64_t)d.T[a] + 1);
-            max_len[a] = std::max(max_len[a], d.size[a]);
-        }
         P->max_iter = std::max(P->max_iter, d.num_iter);
         P->npoints += d.n;
         P->nxlines += H * D;
@@ -1153,13 +1149,10 @@ int plan_create(fb_plan **out, const fb_field *fields, int nfields, int precisio
     cell_prefix.push_back(P->ncells);
     for (int a = 0; a < 3; ++a) lslot[a].push_back(P->lslots[a]);
     for (int a = 0; a < P->dim && !fast; ++a) {
-        P->lgeom[a] = line_geom(max_rect[a], P->max_iter, max_len[a]);
-        if (a && P->lgeom[a].ni) {
-            LineTimes t;
-            for (const FieldDev &d : P->fh)
-                t.add(P->lgeom[a], d.size[a], d.size[0] * d.size[1] * d.size[2] / d.size[a], d.T[a], d.num_iter);
-            if (!t.rings(P->lgeom[a])) P->lgeom[a] = LineGeom();
-        }
+        AxisLines lines_of(a);
+        for (const FieldDev &d : P->fh)
+            lines_of.add(d.size[a], d.size[0] * d.size[1] * d.size[2] / d.size[a], 2 * (int64_t)d.T[a] + 1, d.num_iter);
+        P->lgeom[a] = lines_of.geom();
         const int64_t lines = P->lgeom[a].ni ? kLineSlots / 2 : 1;
         for (const FieldDev &d : P->fh) {
             lwg[a].push_back(P->lwgs[a]);
@@ -2211,7 +2204,9 @@ int fb_accumulate_lines(int tail, int precision, int64_t nlines, int64_t len, in
         if ((rc = launch_zero(d_w, cells * 8, s))) return rc;
         if ((rc = fast_pass_init())) return rc;   // the line kernels' LDS limit
         // line slots, then the workgroups of k_exact_stream
-        const LineGeom g = line_geom(rect_len, num_iter, len);
+        AxisLines lines_of(0);
+        lines_of.add(len, nlines, rect_len, num_iter);
+        const LineGeom g = lines_of.geom();
         const int64_t per = g.ni ? kLineSlots / 2 : 1, nwg = (nlines + per - 1) / per;
         const int64_t pre[4] = {0, 2 * nlines, 0, nwg};
         FB_HIP_CHECK(hipMemcpy(d_pre, pre, sizeof(pre), hipMemcpyHostToDevice));
@@ -2321,12 +2316,9 @@ int fb_convolve_grid(int tail, int precision, int dim, const int64_t *size, cons
         if ((rc = fast_pass_init())) return rc;   // the line kernels' LDS limit
         for (int a = 0; a < dim; ++a) {
             // line slots, then the workgroups of k_exact_stream
-            LineGeom g = line_geom(2 * (int64_t)F.T[a] + 1, num_iter, F.size[a]);
-            if (a && g.ni) {
-                LineTimes t;
-                t.add(g, F.size[a], nl[a], F.T[a], num_iter);
-                if (!t.rings(g)) g = LineGeom();
-            }
+            AxisLines lines_of(a);
+            lines_of.add(F.size[a], nl[a], 2 * (int64_t)F.T[a] + 1, num_iter);
+            const LineGeom g = lines_of.geom();
             const int64_t per = g.ni ? kLineSlots / 2 : 1, nwg = (nl[a] + per - 1) / per;
             const int64_t pre[4] = {0, 2 * nl[a], 0, nwg};
             FB_HIP_CHECK(hipMemcpy(d_pre, pre, sizeof(pre), hipMemcpyHostToDevice));

@@ -189,54 +189,6 @@ inline LineGeom line_geom(int64_t max_rect, int max_iter, int64_t max_len)
     return g;
 }
 
-// Whether an axis' lines go through LDS rings (k_exact_stream) or to a thread each (k_exact_lines).  A
-// ring pass takes its ticks per workgroup of 8 lines, the blocks of a line and the iterations' lag, as
-// often as workgroups follow each other on a CU; a line of one block pays for the lag alone.  A thread
-// per line runs every iteration over memory, and needs many neighbouring lines to hide its chain of
-// dependent steps.  So short columns of large grids are left to the threads: z lines of 1000x1000x6 at 4
-// iterations 1991 us through rings, 209 by threads, of 512x512x16 474 and 141, y lines of 2000 fields of
-// 30x20 167 and 71; but 2400x1200 (T = 27) 58 and 300, z lines of 151x133x61 64 and 74.  Both times are
-// estimated from what 516 shapes of lines of up to 256 nodes measured (2000 to 512000 lines, T = 0 to 70, 1
-// to 8 iterations; the estimates are within 15 and 22 % of the mean); the threads are taken where theirs is
-// less than 0.7 of the rings', where no shape measured lost by it.  Longer lines keep the rings, which were
-// at most 1.25 times slower there and mostly faster.  x lines always take the rings: a thread's accesses
-// along x are strided.  So do plans whose cells are no launch's work-items (2^32).
-class LineTimes {
-public:
-    void add(const LineGeom &g, int64_t len, int64_t lines, int T, int num_iter)
-    {
-        const int64_t wgs = (lines + kLineSlots / 2 - 1) / (kLineSlots / 2);
-        auto launch = [&](int ni) {
-            return ((len + kLineStep - 1) / kLineStep + ni * (2 + T / kLineStep) + 1 + 7) / 8 * 8;
-        };
-        const int rest = num_iter % g.ni;
-        const int64_t ticks = num_iter / g.ni * launch(g.ni) + (rest ? launch(rest) : 0);
-        ticks_ = ticks > ticks_ ? ticks : ticks_;
-        wg_ticks_ += (double)wgs * ticks;
-        lds_ += (double)wgs * g.lds;
-        const double steps = (double)num_iter * (len + T);
-        steps_ = steps > steps_ ? steps : steps_;
-        // an odd number of iterations ends with a copy
-        cells_ += (len * lines + 63) / 64 * 64;
-        cell_us_ += (double)len * lines * (5.9e-6 + (5.2e-6 + 0.1e-6 * T) * (num_iter + (num_iter & 1)));
-        len_ = len > len_ ? len : len_;
-    }
-    bool rings(const LineGeom &g) const
-    {
-        if (len_ > 256 || cells_ > 0xFFFFFF00ll) return true;
-        const int waves = (g.ni + 64 / kLineSlots - 1) / (64 / kLineSlots) + 3;
-        const int by_lds = kLineLdsMax / (int)g.lds, by_waves = 16 / waves;   // 4 waves to a SIMD: registers
-        const double resident = 256.0 * (by_lds < by_waves ? by_lds : by_waves);
-        const double rounds = wg_ticks_ / resident;
-        const double ring_us = 8.0 + 0.69 * (rounds > ticks_ ? rounds : ticks_) + 28e-6 / 256 * lds_;
-        return 19.0 + 0.08 * steps_ + cell_us_ >= 0.7 * ring_us;
-    }
-
-private:
-    int64_t ticks_ = 0, cells_ = 0, len_ = 0;
-    double wg_ticks_ = 0, lds_ = 0, steps_ = 0, cell_us_ = 0;
-};
-
 // FP64 injection: one sorted entry's record (k_field_sort, k_inject_records), in list order.
 struct InjectRec {
     int x;              // base column

@@ -1,5 +1,5 @@
-"""FP64 line passes on both sides of the rule between LDS rings and a thread per line (LineTimes): the
-oracle's bits, and short columns of a large grid in a time that fits their bytes."""
+"""FP64 line passes on both sides of the rules between LDS rings, of more or fewer iterations to a launch, and a
+thread per line (AxisLines): the oracle's bits, and short columns of a large grid in a time that fits their bytes."""
 import numpy as np
 import pytest
 
@@ -32,7 +32,9 @@ def _check(orc, fields, seed):
 # columns of 6 to 24 nodes in grids large and small; odd counts of iterations end in the other buffer
 @pytest.mark.parametrize('size,num_iter,halves', [
     ((1001, 503, 6), 4, (1, 1, 1)), ((601, 6, 301), 5, (1, 1, 1)), ((300, 299, 16), 1, (2, 2, 2)),
-    ((5, 301, 299), 4, (1, 1, 1)), ((100001, 12), 3, (1, 2)), ((70000, 24), 8, (2, 7)), ((40, 31, 6), 4, (1, 1, 1))])
+    ((5, 301, 299), 4, (1, 1, 1)), ((6, 501, 333), 9, (0, 1, 1)), ((16, 101, 307), 8, (3, 1, 1)),
+    ((17, 101, 307), 8, (3, 1, 1)), ((40, 70001), 8, (2, 1)), ((64, 401, 250), 6, (2, 2, 30)),
+    ((100001, 12), 3, (1, 2)), ((70000, 24), 8, (2, 7)), ((40, 31, 6), 4, (1, 1, 1))])
 def test_short_columns_bitwise(orc, size, num_iter, halves):
     _check(orc, [_field(size, 400, num_iter, halves)], size[0])
 
@@ -50,11 +52,9 @@ def test_mixed_iterations_bitwise(orc, halves):
     _check(orc, [_field(size, 200, k, halves) for k in (3, 8, 9, 1, 12)], 11)
 
 
-def test_short_columns_time():
-    """z lines of 6 nodes: through rings they took 34 times the x lines of the same cells."""
-    f = _field((1000, 1000, 6), 2000, 4, (1, 1, 1))
+def _times(f):
     rng = np.random.default_rng(1)
-    pts = hip.DeviceArray.from_numpy(rng.uniform(0.0, 1.0, (f['n'], 3)) * np.asarray(f['size']))
+    pts = hip.DeviceArray.from_numpy(rng.uniform(0.0, 1.0, (f['n'], len(f['size']))) * np.asarray(f['size']))
     val = hip.DeviceArray.from_numpy(rng.normal(0.0, 1.0, f['n']))
     batch = BarnesBatch([f], precision='fp64')
     out = hip.DeviceArray((batch.total_out,), np.float32)
@@ -66,4 +66,16 @@ def test_short_columns_time():
         s.synchronize()
         for k, ms in batch.stage_times().items():
             best[k] = min(best.get(k, ms), ms)
+    return best
+
+
+def test_short_columns_time():
+    """z lines of 6 nodes: through rings they took 34 times the x lines of the same cells."""
+    best = _times(_field((1000, 1000, 6), 2000, 4, (1, 1, 1)))
     assert best['lines_z'] + best['finalize'] < 12.0 * best['lines_x']
+
+
+def test_short_rows_time():
+    """x lines of 30 nodes at 8 iterations: all in one launch they took 5.4 times as long as at 4."""
+    x = [_times(_field((30, 128000), 2000, it, (1, 1)))['lines_x'] for it in (4, 8)]
+    assert x[1] < 3.5 * x[0]
