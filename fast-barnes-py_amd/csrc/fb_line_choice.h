@@ -17,7 +17,8 @@ namespace fb {
 // neighbouring lines to hide its chain of dependent steps, so the shortest lines of large grids are left to the
 // threads: z lines of 1000x1000x6 at 4 iterations 1991 us through rings, 209 by threads, of 512x512x16 474
 // and 141; but of 151x133x61 64 and 74.  Along x its accesses are strided and cost more the longer the lines:
-// 128000 lines of 6 nodes at 8 iterations 1034 and 59, of 12 1008 and 252, of 22 1053 and 860.
+// 128000 lines of 6 nodes at 8 iterations 1034 and 59, of 12 1008 and 252, of 22 1053 and 860 (all iterations in
+// one launch; of 30 nodes 1008 so, 350 in launches of fewer).
 //
 // The times are estimated, from a least-squares fit to what was measured of 2260 ring passes (lines of 6 to 2400
 // nodes, 1000 to 400000 of them, T = 0 to 100, 2 to 12 iterations of which 1 to 8 to a launch; 17 % off

@@ -656,13 +656,12 @@ int launch_field_sort(const FieldDev *d_fields, const int64_t *d_pt_prefix, int 
             else launch(k_field_sort<3, false, T>, T, zero_wgs);
         }
     };
-    // One workgroup of 1024 threads runs on a CU at a time.  Fields of few rows and up to 1024 points are
-    // done as soon by 256 threads (1000 points on 60x40: one field 10.0 us of 1024 threads and 9.1 of 256, 200
-    // fields 13.4 and 12.6); up to 2048 points (one field of 2000 11.5 and 11.8 us) where there are more
-    // fields than CUs (300 fields 24.8 and 20.0).  2000 fields of 50 points on 30x20: 47.8 us of 1024
-    // threads, 14.3 of 256; zero fill, keys and sort in launches of their own took 31.5.
+    // One workgroup of 1024 threads runs on a CU at a time.  Where there are more fields than CUs, small ones
+    // take 256 threads each: 2000 fields of 50 points on 30x20 nodes 47.8 -> 14.3 us (zero fill, keys and sort
+    // in launches of their own took 31.5), 300 fields of 2000 points 24.8 -> 20.0.  Fewer fields gain a tenth
+    // by it, but points crowded into few buckets, for the bitonic network, lose: one field of 406 12.5 -> 17.8.
     constexpr int kSmall = 256;
-    if (max_n <= kSmall * (nfields > 256 ? kSortPerThread : kSortPerThread / 2) && max_rows <= kSmall * kSortPerThread)
+    if (nfields > 256 && max_n <= kSmall * kSortPerThread && max_rows <= kSmall * kSortPerThread)
         run(std::integral_constant<int, kSmall>());
     else
         run(std::integral_constant<int, kLocalSortThreads>());

@@ -1,5 +1,5 @@
 """The sort of many small fields (k_field_sort of 256 threads): the same bits as each field alone, whose sort
-takes 1024 threads from 1025 points or rows on, and as few rounds of workgroups as there are."""
+takes 1024 threads, and as few rounds of workgroups as there are."""
 import numpy as np
 import pytest
 
