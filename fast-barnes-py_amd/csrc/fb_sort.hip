@@ -49,11 +49,12 @@ __device__ __forceinline__ uint32_t block_before(uint32_t v, uint32_t *wsum, uin
 // ---- scan ----------------------------------------------------------------
 
 // out = exclusive scan of in within each tile of kTile words, and tiles[t] = the sum of all tiles before tile
-// t: up to kFewTiles tiles each workgroup sums the words before its own, which spares a launch; beyond that
-// tiles[t] is left the sum of tile t, which k_scan_sums makes it of.  (In one launch, the workgroup that ends
-// last taking the sums, each workgroup's release before its count writes back its L2: 50 ns a tile, 98 us
-// for 2 million rows and 10.9 for 200 thousand; two launches take 9.1 and 5.6.)
-constexpr int kFewTiles = 16;
+// t: up to kFewTiles tiles each workgroup sums the words before its own, which spares a launch (16 tiles 4.0 us,
+// 33 5.1, 64 7.2; two launches 3.0 + 3.0 and the gap between them); beyond that tiles[t] is left the sum of
+// tile t, which k_scan_sums makes it of.  (In one launch, the workgroup that ends last taking the sums, each
+// workgroup's release before its count writes back its L2: 50 ns a tile, 98 us for 2 million rows and 10.9 for
+// 200 thousand; two launches take 9.1 and 5.6.)
+constexpr int kFewTiles = 48;
 
 __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
                                                          int64_t n, uint32_t *__restrict__ tiles)
@@ -62,22 +63,27 @@ __global__ __launch_bounds__(kThreads) void k_scan_tiles(const uint32_t *__restr
     const int tid = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)tid * kItems;
     uint32_t v[kItems] = {}, sum = 0, total, before = 0;
-    const bool few = gridDim.x <= kFewTiles;
-    if (few) {
-        uint32_t pre = 0;
-#pragma unroll 4
-        for (int t = 0; t < (int)blockIdx.x; ++t) {
-            const uint4 x = reinterpret_cast<const uint4 *>(in + (int64_t)t * kTile)[tid];
-            pre += x.x + x.y + x.z + x.w;
-        }
-        block_before(pre, wpre, before);
-    }
     if (base + kItems <= n) {
         const uint4 x = *reinterpret_cast<const uint4 *>(in + base);
         v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
     } else {
 #pragma unroll
         for (int i = 0; i < kItems; ++i) v[i] = base + i < n ? in[base + i] : 0u;
+    }
+    const bool few = gridDim.x <= kFewTiles;
+    if (few) {
+        constexpr int kLoads = 16;   // in flight
+        uint32_t pre = 0;
+        for (int t0 = 0; t0 < (int)blockIdx.x; t0 += kLoads) {
+            uint4 x[kLoads];
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u)
+                x[u] = t0 + u < (int)blockIdx.x ? reinterpret_cast<const uint4 *>(in + (int64_t)(t0 + u) * kTile)[tid]
+                                                : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) pre += x[u].x + x[u].y + x[u].z + x[u].w;
+        }
+        block_before(pre, wpre, before);
     }
 #pragma unroll
     for (int i = 0; i < kItems; ++i) sum += v[i];

@@ -9,8 +9,10 @@ from fastbarnes.batched import BarnesBatch
 pytestmark = pytest.mark.gpu
 
 
-# rows around 16 tiles (beyond, k_scan_sums), 4096 tiles (a round of it) and 512 * 1024 (rows 16 by 16)
-@pytest.mark.parametrize('rows', [8193, (1 << 14) - 1, 1 << 14, (1 << 14) + 1, (1 << 19) - 1, (1 << 19) + 1, (1 << 19) + 40000, (1 << 22) - 1,
+# rows around 16 tiles (loads in flight), 48 (beyond, k_scan_sums), 4096 (a round of it) and 512 * 1024 (rows 16
+# by 16)
+@pytest.mark.parametrize('rows', [8193, (1 << 14) - 1, 1 << 14, (1 << 14) + 1, (1 << 14) + 1025, 48 * 1024 - 1, 48 * 1024,
+                                  48 * 1024 + 1, (1 << 19) - 1, (1 << 19) + 1, (1 << 19) + 40000, (1 << 22) - 1,
                                   (1 << 22) + 2050])
 def test_many_rows_bitwise(orc, rows):
     rng = np.random.default_rng(rows)
