@@ -44,7 +44,7 @@ public:
     LineGeom geom() const
     {
         const LineGeom most = line_geom(max_rect_, max_iter_, max_len_);
-        if (!most.ni) return most;
+        if (!most.ni || max_iter_ > kMostIter) return most;
         const double most_us = rings(most);
         LineGeom g = most;
         double us = most_us;
@@ -63,6 +63,7 @@ public:
     }
 
 private:
+    static constexpr int kMostIter = 1000;   // iterations up to which the estimates, a sum over launches, are formed
     struct Lines {
         int64_t len, lines, T;
         int num_iter;
